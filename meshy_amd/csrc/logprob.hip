@@ -6,8 +6,9 @@
 // at trainer.py:414-428 and logsumexp(z) - sum(softmax(z) * z) at
 // trainer.py:430-449, and the chunked gather of gather_logprobs,
 // meshy/backend/titan/topk_loss.py:35-57): one workgroup streams one row of
-// V logits from HBM exactly once with 16-byte loads and keeps, per lane, the
-// online (m, s, t) state of rowstream.h, updated once per register tile.
+// V logits from HBM exactly once with 16-byte loads, whatever the row's
+// alignment, and keeps, per lane, the online (m, s, t) state of rowstream.h,
+// updated once per register tile.
 // Lanes and waves merge their triples; then
 //     lse = m + ln s,  logp_k = z_{y_k} - lse,  H = ln 2 * (log2 s - t / s)
 // for the row's n_ids gather ids y_k.  No fp32 copy of the logits is made.
@@ -93,31 +94,34 @@ __device__ __forceinline__ void accumulate_exact(v4u (&v)[U], float& m, float& s
     accumulate(z, m, s, t);
 }
 
-// Vector path: row base 16-byte aligned.  NT threads per row, U 16-byte loads
-// in flight per thread per tile.  A lane's first tile sets its running max;
-// later tiles are accumulated against it (accumulate_at) and take the tile
-// max only when an element lies more than 44 above it.  The chunks left after
-// the full tiles form one predicated tile.
+// Bound by the read of the logits.  NT threads per row (fwd_threads), U 16-byte
+// loads in flight per thread per tile.  A lane's first tile sets its running max; later tiles are accumulated against it
+// (accumulate_at) and take the tile max only when an element lies more than 44
+// above it.  The chunks left after the full tiles form one predicated tile.
+// The elements outside the row's 16-byte chunks (row_span) are loaded before
+// the first tile and added after the last, one per thread: 4096 rows of 50257
+// logits take 65.6 us (6.28 TB/s) against 81.3 with 2-byte loads throughout.
 template <int NT, int U>
 __global__ __launch_bounds__(NT) void k_lpe_fwd_vec(const uint16_t* __restrict__ logits, int64_t T,
                                                     int64_t V, int64_t stride_b, int64_t stride_t,
                                                     const int64_t* __restrict__ ids, int n_ids,
-                                                    float* __restrict__ logp,
-                                                    float* __restrict__ ent,
+                                                    float* __restrict__ logp, float* __restrict__ ent,
                                                     float* __restrict__ lse_out) {
     const int64_t r = blockIdx.x;
     const uint16_t* row = row_ptr(logits, r, T, stride_b, stride_t);
-    const v4u* row4 = reinterpret_cast<const v4u*>(row);
+    const RowSpan sp = row_span(row, V);
     const int tid = threadIdx.x;
     int64_t y;
     float zy;
     load_id(row, ids, r, n_ids, V, y, zy);
+    bool edge;
+    const int64_t e = edge_element(sp, V, tid, edge);
+    const float z_edge = edge ? bf16_to_f32(row[e]) : 0.f;
 
     float m = kInit, s = 0.f, t = 0.f;
-    const int64_t n8 = V >> 3;
     constexpr int64_t kTile = static_cast<int64_t>(NT) * U;
-    const int64_t n_full = n8 / kTile;
-    const v4u* p = row4 + tid;
+    const int64_t n_full = sp.n8 / kTile;
+    const v4u* p = sp.body + tid;
     for (int64_t it = 0; it < n_full; ++it, p += kTile) {
         v4u v[U];
 #pragma unroll
@@ -130,42 +134,10 @@ __global__ __launch_bounds__(NT) void k_lpe_fwd_vec(const uint16_t* __restrict__
             accumulate_exact(v, m, s, t);
         }
     }
-    const int64_t rem = n8 - n_full * kTile;
-    if (rem > 0) lpe_tail<NT, 1, U>(row4 + n_full * kTile, rem, tid, m, s, t);
-    // Tail elements when V is not a multiple of 8.
-    {
-        const int64_t e = (n8 << 3) + tid;
-        const bool ok = e < V;
-        accumulate_one(ok ? bf16_to_f32(row[e]) : 0.f, ok, m, s, t);
-    }
+    const int64_t rem = sp.n8 - n_full * kTile;
+    if (rem > 0) lpe_tail<NT, 1, U>(sp.body + n_full * kTile, rem, tid, m, s, t);
+    accumulate_one(z_edge, edge, m, s, t);
 
-    block_merge<NT>(m, s, t);
-    finish_row<NT>(r, m, s, t, y, zy, V, n_ids, logp, ent, lse_out);
-}
-
-// Generic path: any alignment and stride, 2-byte coalesced loads.
-template <int NT>
-__global__ __launch_bounds__(NT) void k_lpe_fwd_any(const uint16_t* __restrict__ logits, int64_t T,
-                                                    int64_t V, int64_t stride_b, int64_t stride_t,
-                                                    const int64_t* __restrict__ ids, int n_ids,
-                                                    float* __restrict__ logp,
-                                                    float* __restrict__ ent,
-                                                    float* __restrict__ lse_out) {
-    const int64_t r = blockIdx.x;
-    const uint16_t* row = row_ptr(logits, r, T, stride_b, stride_t);
-    const int tid = threadIdx.x;
-    int64_t y;
-    float zy;
-    load_id(row, ids, r, n_ids, V, y, zy);
-    float m = kInit, s = 0.f, t = 0.f;
-    int64_t e = tid;
-    for (; e + 7 * NT < V; e += 8 * NT) {
-        float z[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) z[u] = bf16_to_f32(row[e + u * NT]);
-        accumulate(z, m, s, t);
-    }
-    for (; e < V; e += NT) accumulate_one(bf16_to_f32(row[e]), true, m, s, t);
     block_merge<NT>(m, s, t);
     finish_row<NT>(r, m, s, t, y, zy, V, n_ids, logp, ent, lse_out);
 }
@@ -308,11 +280,9 @@ __global__ __launch_bounds__(256) void k_lp_bwd_fix(const uint16_t* __restrict__
     out[r * V + y] = __bfloat16_as_ushort(__float2bfloat16(q));
 }
 
-// 256 threads x 8 16-byte loads in flight per tile: the fastest forward shape
-// of a sweep over {64..1024} threads x {2, 4, 8} loads on MI355X.  The flat
-// backward: 256 threads x 4 loads, 65536 workgroups (sweep over 16384..65536
-// workgroups, 2..8 loads).
-constexpr int kFwdThreads = 256;
+// 8 16-byte loads in flight per thread per tile (4 are slower at every size).
+// The flat backward: 256 threads x 4 loads, 65536 workgroups (sweep over
+// 16384..65536 workgroups, 2..8 loads).
 constexpr int kFwdUnroll = 8;
 constexpr int kBwdThreads = 256;
 constexpr int kBwdUnroll = 4;
@@ -337,19 +307,33 @@ bool vector_ok(const void* logits, int64_t stride_b, int64_t stride_t) {
     return (reinterpret_cast<uintptr_t>(logits) % 16 == 0) && (stride_b % 8 == 0) && (stride_t % 8 == 0);
 }
 
+// Threads of a row's workgroup.  Up to 256 rows there is one workgroup per CU
+// at most, and a CU streams in proportion to its loads in flight: 512 threads
+// take 13.0 us for 37 rows of 151936 logits and 16.0 for 256, against 19.1 and
+// 21.1 with 256 threads (1024 threads: 12.4 and 16.3).  From 257 rows on, 256
+// threads spread the rows more evenly (512 rows: 27.4 against 28.1 us; 4096
+// rows of 50257: 65.6 against 72.2, where most of a row is the predicated last
+// tile of 4096 chunks).  Many rows of at least 3 full tiles of 512 threads
+// stream faster with those (4096 rows of 131072: 158.0 against 162.4 us; 16384
+// of 151936: 703 against 714; 4096 of 81920, 2.5 tiles: 102.2 against 103.5).
+int fwd_threads(int64_t n, int64_t V) {
+    return n <= 256 || (n >= 2048 && V >= 3 * 512 * kFwdUnroll * 8) ? 512 : 256;
+}
+
 int launch_fwd(const uint16_t* logits, int64_t rows, int64_t T, int64_t V, int64_t stride_b,
                int64_t stride_t, const int64_t* ids, int n_ids, float* out, float* entropy, float* lse,
                hipStream_t stream, const char* who) {
     const int64_t n = rows * T;
     if (n == 0) return MESHY_OK;
     const dim3 grid(static_cast<unsigned>(n));
-    if (vector_ok(logits, stride_b, stride_t)) {
-        hipLaunchKernelGGL((k_lpe_fwd_vec<kFwdThreads, kFwdUnroll>), grid, dim3(kFwdThreads), 0, stream,
-                           logits, T, V, stride_b, stride_t, ids, n_ids, out, entropy, lse);
-    } else {
-        hipLaunchKernelGGL((k_lpe_fwd_any<kFwdThreads>), grid, dim3(kFwdThreads), 0, stream, logits, T,
-                           V, stride_b, stride_t, ids, n_ids, out, entropy, lse);
-    }
+    auto go = [&](auto kernel, int threads) {
+        hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, stream, logits, T, V, stride_b, stride_t, ids, n_ids, out,
+                           entropy, lse);
+    };
+    if (fwd_threads(n, V) == 512)
+        go(k_lpe_fwd_vec<512, kFwdUnroll>, 512);
+    else
+        go(k_lpe_fwd_vec<256, kFwdUnroll>, 256);
     return check_launch(who);
 }
 

@@ -187,18 +187,45 @@ __device__ __forceinline__ void accumulate_one(float z, bool ok, float& m, float
     t = fmaf(e, x, t);
 }
 
+// Merges each lane's triple with that of the lane kCtrl rotates to it.
+template <int kCtrl>
+__device__ __forceinline__ void merge_dpp(float& m, float& s, float& t) {
+    const float m2 = dpp_f32<kCtrl>(m);
+    const float s2 = dpp_f32<kCtrl>(s);
+    const float t2 = dpp_f32<kCtrl>(t);
+    merge(m, s, t, m2, s2, t2);
+}
+
+// The merge over each 16-lane row through DPP rotations, valid in lane 0 of
+// the row.
+__device__ __forceinline__ void merge_rows16(float& m, float& s, float& t) {
+    merge_dpp<kDppRowRor8>(m, s, t);
+    merge_dpp<kDppRowRor4>(m, s, t);
+    merge_dpp<kDppRowRor2>(m, s, t);
+    merge_dpp<kDppRowRor1>(m, s, t);
+}
+
 // Block-wide merge of the per-lane triples; the result lands in thread 0.
+// Rows of 16 lanes and then the waves' triples go through DPP rotations: with
+// 16 waves a chain of one merge per wave in thread 0 alone took longer than
+// the rest of the merge.
 template <int NT>
 __device__ __forceinline__ void block_merge(float& m, float& s, float& t) {
+    merge_rows16(m, s, t);
+    float mr[4], sr[4], tr[4];
 #pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) {
-        const float m2 = __shfl_xor(m, off, kWave);
-        const float s2 = __shfl_xor(s, off, kWave);
-        const float t2 = __shfl_xor(t, off, kWave);
-        merge(m, s, t, m2, s2, t2);
+    for (int r = 0; r < 4; ++r) {
+        mr[r] = lane_f32(m, 16 * r);
+        sr[r] = lane_f32(s, 16 * r);
+        tr[r] = lane_f32(t, 16 * r);
     }
+    merge(mr[0], sr[0], tr[0], mr[1], sr[1], tr[1]);
+    merge(mr[2], sr[2], tr[2], mr[3], sr[3], tr[3]);
+    m = mr[0], s = sr[0], t = tr[0];
+    merge(m, s, t, mr[2], sr[2], tr[2]);
     if constexpr (NT > kWave) {
         constexpr int kWaves = NT / kWave;
+        static_assert(kWaves <= 16, "the waves' triples are merged in one row of 16 lanes");
         __shared__ float sm[kWaves], ss[kWaves], st[kWaves];
         const int lane = threadIdx.x % kWave;
         const int wid = threadIdx.x / kWave;
@@ -208,11 +235,48 @@ __device__ __forceinline__ void block_merge(float& m, float& s, float& t) {
             st[wid] = t;
         }
         __syncthreads();
-        if (threadIdx.x == 0) {
-#pragma unroll
-            for (int w = 1; w < kWaves; ++w) merge(m, s, t, sm[w], ss[w], st[w]);
+        if (wid == 0) {
+            const bool in = lane < kWaves;
+            m = in ? sm[lane] : kInit;
+            s = in ? ss[lane] : 0.f;
+            t = in ? st[lane] : 0.f;
+            merge_rows16(m, s, t);
         }
     }
+}
+
+// How a row of V logits is streamed: `head` elements up to the first 128-byte
+// boundary, n8 16-byte chunks from there, and `tail` elements after them.
+// Rows start at any element (V odd, strided or offset views), and a wave's
+// 1 KB load instruction then still covers whole 128-byte lines.
+constexpr int kLineElems = 64;  // elements of a 128-byte line
+
+struct RowSpan {
+    const v4u* body;
+    int64_t n8;
+    int head;  // < kLineElems
+    int tail;  // < 8
+};
+
+__device__ __forceinline__ RowSpan row_span(const uint16_t* row, int64_t V) {
+    RowSpan sp;
+    const uintptr_t past = reinterpret_cast<uintptr_t>(row) % (2 * kLineElems);
+    const int64_t to_line = past ? static_cast<int64_t>((2 * kLineElems - past) / 2) : 0;
+    sp.head = static_cast<int>(min(to_line, V));
+    sp.body = reinterpret_cast<const v4u*>(row + sp.head);
+    sp.n8 = (V - sp.head) >> 3;
+    sp.tail = static_cast<int>((V - sp.head) & 7);
+    return sp;
+}
+
+// The element of the row's head or tail that thread tid holds (head elements
+// in threads 0 .., tail elements from thread kLineElems on), and whether it
+// holds one.
+__device__ __forceinline__ int64_t edge_element(const RowSpan& sp, int64_t V, int tid, bool& ok) {
+    const bool in_head = tid < sp.head;
+    const bool in_tail = tid >= kLineElems && tid < kLineElems + sp.tail;
+    ok = in_head || in_tail;
+    return in_tail ? V - sp.tail + (tid - kLineElems) : (in_head ? tid : 0);
 }
 
 __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
