@@ -293,8 +293,7 @@ int meshy_zero_variance_groups_host(const double* raw_rewards, int64_t n_rewards
  * _chunk_entropy (trainer.py:430-449: logsumexp - sum softmax * z).
  *
  * logits element (b, t, v) lives at logits[b*stride_b + t*stride_t + v]
- * (strides in elements; stride_b, stride_t multiples of 8 and logits 16-byte
- * aligned take the vector path, anything else the unaligned path).
+ * (strides in elements; rows may start at any element).
  * labels is contiguous [rows * T]; a label of -100 (cross_entropy's default
  * ignore_index) gives logp = 0; a label outside [0, V) gives NaN.
  * Outputs are contiguous [rows * T] fp32; each may be NULL.  lse is what the
@@ -310,8 +309,9 @@ int meshy_logprob_entropy_fwd(const uint16_t* logits, int64_t rows, int64_t T, i
  * written as bf16 into a contiguous [rows * T, V] buffer.  Ignored labels
  * (-100) give a zero row, labels outside [0, V) a NaN row.  This is the
  * gradient torch autograd produces for the reference's checkpointed
- * -cross_entropy chunk (trainer.py:504-517).  The workspace holds two floats
- * per row (meshy_logprob_bwd_workspace_size(rows * T) bytes).
+ * -cross_entropy chunk (trainer.py:504-517).  The call must pass a workspace
+ * of meshy_logprob_bwd_workspace_size(rows * T) bytes, which it does not touch
+ * (the backward is one pass).
  */
 size_t meshy_logprob_bwd_workspace_size(int64_t n_rows);
 int meshy_logprob_bwd(const uint16_t* logits, int64_t rows, int64_t T, int64_t V,
@@ -324,11 +324,9 @@ int meshy_logprob_bwd(const uint16_t* logits, int64_t rows, int64_t T, int64_t V
  * reference: it is for callers that cannot allocate device memory or pass a
  * workspace (code under HIP graph capture, tight training or serving loops,
  * harnesses that forbid hipMalloc).  Same arguments, kernels and results as
- * meshy_logprob_bwd; its two floats per row live in a static device array of
- * MESHY_NOALLOC_MAX_ROWS rows (2 MiB, one copy per GPU, held until the
- * process ends).  rows * T above that limit returns MESHY_ESPACE.  The call
- * allocates and frees nothing.  Calls that overlap on one GPU (on different
- * streams) share that array and race; calls on one stream are ordered.
+ * meshy_logprob_bwd.  rows * T above MESHY_NOALLOC_MAX_ROWS returns
+ * MESHY_ESPACE.  The call allocates and frees nothing and shares nothing with
+ * other calls.
  */
 #define MESHY_NOALLOC_MAX_ROWS 262144
 int meshy_logprob_bwd_noalloc(const uint16_t* logits, int64_t rows, int64_t T, int64_t V,

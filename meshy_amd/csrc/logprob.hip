@@ -14,20 +14,18 @@
 // for the row's n_ids gather ids y_k.  No fp32 copy of the logits is made.
 //
 // Backward: grad[r, v] = sum_k g[r,k] onehot(y_k)[v] - G_r exp(z[r, v] - lse[r]),
-// G_r = sum_k g[r,k], written as bf16 in three launches: a per-row prep
-// (-G_r and -lse_r log2 e into the workspace), the streaming pass of the
-// softmax term, and a fixup of the n_ids one-hot positions.  The streaming
-// pass walks the flattened [rows * V] grid with a grid-stride loop when the
-// logits are contiguous: on MI355X that order writes 8 % faster than one
-// workgroup per row.
+// G_r = sum_k g[r,k], written as bf16 in one pass over the flattened
+// [rows * V] gradient with a grid-stride loop: on MI355X that order writes 8 %
+// faster than one workgroup per row.
 #include <algorithm>
-#include <atomic>
-#include <mutex>
+#include <type_traits>
 
 #include "rowstream.h"
 
 namespace meshy {
 namespace {
+
+constexpr int kMaxIds = 256;  // gather ids per row (one thread each)
 
 // thread 0: lse, entropy, and (with one id) the log-prob.
 __device__ __forceinline__ float id_logp(int64_t y, float zy, float lse, int64_t V) {
@@ -144,150 +142,269 @@ __global__ __launch_bounds__(NT) void k_lpe_fwd_vec(const uint16_t* __restrict__
 
 // ---------------------------------------------------------------- backward
 
-// Per row: ng = -G (NaN when an id is neither -100 nor in [0, V)) and
-// nl = -lse * log2 e.
-__global__ __launch_bounds__(256) void k_lp_bwd_prep(const int64_t* __restrict__ ids, int n_ids,
-                                                     const float* __restrict__ lse,
-                                                     const float* __restrict__ grad, int64_t n_rows,
-                                                     int64_t V, float* __restrict__ ng,
-                                                     float* __restrict__ nl) {
-    const int64_t r = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-    if (r >= n_rows) return;
-    float G = 0.f;
-    bool bad = false;
-    for (int k = 0; k < n_ids; ++k) {
-        const int64_t y = ids[r * n_ids + k];
-        if (y == kIgnoreIndex) continue;
-        if (y < 0 || y >= V) bad = true;
-        G += grad[r * n_ids + k];
+struct BwdArgs {
+    const uint16_t* logits;
+    int64_t T, V, stride_b, stride_t;
+    int64_t row0;       // the launch's first row (a multiple of 8); the arrays below start at it
+    int64_t n_elems;    // of the launch's gradient
+    uint32_t n_chunks;  // ceil(n_elems / 8)
+    double inv_v;
+    int n_ids;
+    const int64_t* ids;
+    const float* lse;
+    const float* grad_logp;
+    uint16_t* out;
+};
+
+__device__ __forceinline__ uint16_t bf16_bits(float x) { return __bfloat16_as_ushort(__float2bfloat16(x)); }
+
+// The k-th id of a row (-1 where it adds nothing) and its gradient; returns
+// whether it is neither -100 nor in [0, V).
+__device__ __forceinline__ bool row_id(const BwdArgs& a, int64_t r, int k, int64_t& y, float& g) {
+    y = a.ids[r * a.n_ids + k];
+    g = a.grad_logp[r * a.n_ids + k];
+    const bool ignored = y == kIgnoreIndex;
+    const bool bad = !ignored && (y < 0 || y >= a.V);
+    if (ignored) g = 0.f;
+    if (ignored || bad) y = -1;
+    return bad;
+}
+
+// What the pass needs of a row: ng = -G (NaN when an id is out of range),
+// nl = -lse log2 e, and its ids with their gradients, NB 64-id blocks with one
+// id per lane.  NB = 0: one id, the same in every lane.
+template <int NB>
+struct BwdRow {
+    float ng, nl;
+    int64_t y[NB ? NB : 1];
+    float g[NB ? NB : 1];
+};
+
+// Row r, wave-uniform; all 64 lanes active.
+template <int NB>
+__device__ __forceinline__ BwdRow<NB> bwd_row(const BwdArgs& a, int64_t r) {
+    BwdRow<NB> w;
+    w.nl = -a.lse[r] * kLog2e;
+    if constexpr (NB == 0) {
+        const bool bad = row_id(a, r, 0, w.y[0], w.g[0]);
+        w.ng = bad ? __builtin_nanf("") : -w.g[0];
+    } else {
+        bool bad = false;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const int k = b * kWave + threadIdx.x % kWave;
+            const bool over = row_id(a, r, min(k, a.n_ids - 1), w.y[b], w.g[b]);
+            bad |= over && k < a.n_ids;
+            if (k >= a.n_ids) w.y[b] = -1, w.g[b] = 0.f;
+        }
+        float G = 0.f;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) G += wave_sum(w.g[b]);
+        w.ng = __ballot(bad) ? __builtin_nanf("") : -G;
     }
-    ng[r] = bad ? __builtin_nanf("") : -G;
-    nl[r] = -lse[r] * kLog2e;
+    return w;
 }
 
-__device__ __forceinline__ v4u softmax_term8(v4u v, float ng, float nl) {
-    float z[8];
-    const v4u vv[1] = {v};
-    unpack(vv, z);
-    float q[8];
+// q[0 .. 7] += the row's one-hot terms among the 512 elements of the wave whose
+// first is the row's column lo: lane l holds columns lo + 8 l .. lo + 8 l + 7.
+// Duplicate ids add in order of k.
+template <int NB>
+__device__ __forceinline__ void add_onehot(const BwdRow<NB>& w, int64_t lo, float (&q)[8]) {
+    const int lane = threadIdx.x % kWave;
+    auto add = [&](int off, float g) {  // wave-uniform offset from lo
+        const float gl = lane == off >> 3 ? g : 0.f;
 #pragma unroll
-    for (int k = 0; k < 8; ++k) q[k] = ng * fast_exp2(fmaf(z[k], kLog2e, nl));
-    v4u o;
-    o.x = pack_bf16x2(q[0], q[1]);
-    o.y = pack_bf16x2(q[2], q[3]);
-    o.z = pack_bf16x2(q[4], q[5]);
-    o.w = pack_bf16x2(q[6], q[7]);
-    return o;
-}
-
-// Row index of 16-byte chunk c of a contiguous [rows, V] grid (n8 chunks per
-// row): a double-precision estimate corrected by one step.
-__device__ __forceinline__ uint32_t row_of_chunk(uint32_t c, uint32_t n8, double inv_n8) {
-    uint32_t r = static_cast<uint32_t>(static_cast<double>(c) * inv_n8);
-    if (r * n8 > c) --r;
-    else if ((r + 1) * n8 <= c) ++r;
-    return r;
-}
-
-// Streaming pass over contiguous logits [rows, V], V % 8 == 0: grid-stride
-// over the n_chunks 16-byte chunks, U loads in flight per thread.
-template <int NT, int U>
-__global__ __launch_bounds__(NT) void k_lp_bwd_flat(const v4u* __restrict__ z4, uint32_t n8,
-                                                    uint32_t n_chunks, double inv_n8,
-                                                    const float* __restrict__ ng,
-                                                    const float* __restrict__ nl,
-                                                    v4u* __restrict__ g4) {
-    uint32_t i = blockIdx.x * (NT * U) + threadIdx.x;
-    const uint32_t stride = gridDim.x * (NT * U);
-    for (; i + (U - 1) * NT < n_chunks; i += stride) {
-        v4u v[U];
+        for (int k = 0; k < 8; ++k)
+            if ((off & 7) == k) q[k] += gl;
+    };
 #pragma unroll
-        for (int u = 0; u < U; ++u) v[u] = __builtin_nontemporal_load(z4 + i + u * NT);
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const uint32_t c = i + u * NT;
-            const uint32_t r = row_of_chunk(c, n8, inv_n8);
-            __builtin_nontemporal_store(softmax_term8(v[u], ng[r], nl[r]), g4 + c);
+    for (int b = 0; b < (NB ? NB : 1); ++b) {
+        const int64_t off = w.y[b] - lo;
+        const bool in = w.y[b] >= 0 && static_cast<uint64_t>(off) < 8 * kWave;
+        if constexpr (NB == 0) {
+            if (in) add(static_cast<int>(off), w.g[0]);
+        } else {
+            uint64_t hit = __ballot(in);
+            while (hit) {
+                const int l = __builtin_ctzll(hit);
+                hit &= hit - 1;
+                add(__builtin_amdgcn_readlane(static_cast<int>(off), l), lane_f32(w.g[b], l));
+            }
         }
     }
-    for (; i < n_chunks; i += NT) {
-        const uint32_t r = row_of_chunk(i, n8, inv_n8);
-        __builtin_nontemporal_store(softmax_term8(__builtin_nontemporal_load(z4 + i), ng[r], nl[r]), g4 + i);
+}
+
+// Row and column of element e of the launch's [rows, V] gradient: a
+// double-precision estimate (e is exact in it) corrected by one step.
+__device__ __forceinline__ void locate(const BwdArgs& a, int64_t e, uint32_t& r, int64_t& pos) {
+    r = static_cast<uint32_t>(static_cast<double>(e) * a.inv_v);
+    pos = e - r * a.V;
+    if (pos < 0) {
+        --r;
+        pos += a.V;
+    } else if (pos >= a.V) {
+        ++r;
+        pos -= a.V;
     }
 }
 
-// Streaming pass, one workgroup per row: strided logits with 16-byte aligned
-// rows and V % 8 == 0.
-template <int NT, int U>
-__global__ __launch_bounds__(NT) void k_lp_bwd_rows(const uint16_t* __restrict__ logits, int64_t T,
-                                                    int64_t V, int64_t stride_b, int64_t stride_t,
-                                                    const float* __restrict__ ng,
-                                                    const float* __restrict__ nl,
-                                                    uint16_t* __restrict__ grad) {
-    const int64_t r = blockIdx.x;
-    const v4u* row4 = reinterpret_cast<const v4u*>(row_ptr(logits, r, T, stride_b, stride_t));
-    v4u* grow4 = reinterpret_cast<v4u*>(grad + r * V);
-    const float g = ng[r], l = nl[r];
-    const int64_t n8 = V >> 3;
-    int64_t c = threadIdx.x;
-    for (; c + (U - 1) * NT < n8; c += NT * U) {
-        v4u v[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) v[u] = __builtin_nontemporal_load(row4 + c + u * NT);
-#pragma unroll
-        for (int u = 0; u < U; ++u) __builtin_nontemporal_store(softmax_term8(v[u], g, l), grow4 + c + u * NT);
+// The 8 logits of a chunk that one 16-byte load does not cover, element by
+// element (elements past the end repeat the last one).
+template <bool kContig>
+__device__ __forceinline__ v4u load_chunk_elements(const BwdArgs& a, int64_t e0) {
+    uint64_t half[2] = {0, 0};
+#pragma unroll 1
+    for (int k = 0; k < 8; ++k) {
+        const int64_t e = min(e0 + k, a.n_elems - 1);
+        uint64_t h;
+        if constexpr (kContig) {
+            h = a.logits[a.row0 * a.V + e];
+        } else {
+            uint32_t r;
+            int64_t pos;
+            locate(a, e, r, pos);
+            h = row_ptr(a.logits, a.row0 + r, a.T, a.stride_b, a.stride_t)[pos];
+        }
+        h <<= 16 * (k & 3);
+        half[0] |= k < 4 ? h : 0;
+        half[1] |= k < 4 ? 0 : h;
     }
-    for (; c < n8; c += NT) __builtin_nontemporal_store(softmax_term8(__builtin_nontemporal_load(row4 + c), g, l), grow4 + c);
+    return v4u{static_cast<uint32_t>(half[0]), static_cast<uint32_t>(half[0] >> 32), static_cast<uint32_t>(half[1]),
+               static_cast<uint32_t>(half[1] >> 32)};
 }
 
-// Streaming pass, generic: any alignment, stride and V.
-template <int NT>
-__global__ __launch_bounds__(NT) void k_lp_bwd_any(const uint16_t* __restrict__ logits, int64_t T,
-                                                   int64_t V, int64_t stride_b, int64_t stride_t,
-                                                   const float* __restrict__ ng,
-                                                   const float* __restrict__ nl,
-                                                   uint16_t* __restrict__ grad) {
+// 16 bytes at any element (the hardware's global loads need no alignment).
+typedef v4u v4u_any __attribute__((aligned(2)));
+
+// A wave-uniform value moved to scalar registers.
+__device__ __forceinline__ int64_t uniform_i64(int64_t x) {
+    return (static_cast<int64_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(x >> 32))) << 32) |
+           static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(x)));
+}
+
+// The whole backward in one pass over the 16-byte chunks of the contiguous
+// gradient, bound by its read and write: 5.95 TB/s on [8192, 151936] (837 us
+// with the forward's 358 in one loop; 861 in three launches), 5.99 on
+// [8192, 50257] (275 us; 610 with 2-byte accesses).  Each wave takes U groups
+// of 64 consecutive chunks, its U loads per lane in flight together, and the
+// grid covers the chunks once: U = 2 takes 1160 us forward and backward on
+// [8192, 151936], U = 4 and 8 1205 and 1243, a grid-stride loop of 65536
+// workgroups 1200; going from the last chunk to the first (towards what the
+// forward read last) changes nothing.  kContig: the logits are contiguous too,
+// so a chunk is 8 consecutive elements of both whatever V is; other logits are
+// read at their row's address.  Most waves' U groups lie in one row, whose
+// factors and ids are then wave-uniform: the wave reads them itself while its
+// logits are in flight, which costs less than the two passes over the rows
+// (factors before, one-hot terms after) that it replaces.  Waves that hold a
+// row's end take each of their rows in turn.
+template <int NT, int U, int NB, bool kContig>
+__global__ __launch_bounds__(NT) void k_lp_bwd_flat(BwdArgs a) {
+    const int lane = threadIdx.x % kWave;
+    const uint32_t c0 = blockIdx.x * (NT * U) + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) * (kWave * U);
+    if (c0 >= a.n_chunks) return;
+    const int64_t last = a.n_chunks - 1;
+    const int64_t e0 = static_cast<int64_t>(c0) * 8;
+    uint32_t r;
+    int64_t lo;
+    locate(a, e0, r, lo);
+    r = __builtin_amdgcn_readfirstlane(r);
+    lo = uniform_i64(lo);
+    const uint16_t* row = row_ptr(a.logits, a.row0 + r, a.T, a.stride_b, a.stride_t);
+    // Lanes past the end repeat the last whole chunk; a chunk that no one load
+    // covers is read again below.
+    v4u v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int64_t c = min<int64_t>(c0 + u * kWave + lane, last);
+        if constexpr (kContig) {
+            const int64_t whole = c * 8 + 8 <= a.n_elems ? c : 0;
+            v[u] = __builtin_nontemporal_load(reinterpret_cast<const v4u*>(a.logits + a.row0 * a.V) + whole);
+        } else {
+            const int64_t p = lo + (c - c0) * 8;
+            v[u] = __builtin_nontemporal_load(reinterpret_cast<const v4u_any*>(row + (p + 8 <= a.V ? p : 0)));
+        }
+    }
+    const BwdRow<NB> w0 = bwd_row<NB>(a, r);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int64_t c = static_cast<int64_t>(c0) + u * kWave + lane;
+        const int64_t e = c * 8;
+        if (kContig ? e + 8 > a.n_elems : lo + (e - e0) + 8 > a.V) {
+            if (c <= last) v[u] = load_chunk_elements<kContig>(a, e);
+        }
+        float z[8], q[8];
+        const v4u vv[1] = {v[u]};
+        unpack(vv, z);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) q[k] = w0.ng * fast_exp2(fmaf(z[k], kLog2e, w0.nl));
+        add_onehot(w0, lo + u * 8 * kWave, q);
+        // Elements of the rows that start inside this group.
+        const int64_t end = min<int64_t>(e0 + (u + 1) * 8 * kWave, a.n_elems);
+        for (uint32_t rr = r + 1; rr * a.V < end; ++rr) {
+            const int64_t at = e - rr * a.V;  // the lane's column in row rr
+            const BwdRow<NB> w = bwd_row<NB>(a, rr);
+            float x[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) x[k] = w.ng * fast_exp2(fmaf(z[k], kLog2e, w.nl));
+            add_onehot(w, e0 + u * 8 * kWave - rr * a.V, x);
+#pragma unroll
+            for (int k = 0; k < 8; ++k) q[k] = at + k >= 0 ? x[k] : q[k];
+        }
+        if (c <= last) {
+            v4u o;
+            o.x = pack_bf16x2(q[0], q[1]);
+            o.y = pack_bf16x2(q[2], q[3]);
+            o.z = pack_bf16x2(q[4], q[5]);
+            o.w = pack_bf16x2(q[6], q[7]);
+            if (e + 8 <= a.n_elems) {
+                __builtin_nontemporal_store(o, reinterpret_cast<v4u*>(a.out) + c);
+            } else {
+                for (int k = 0; e + k < a.n_elems; ++k) a.out[e + k] = bf16_bits(q[k]);
+            }
+        }
+    }
+}
+
+// One workgroup per row, an element per thread at a time: short rows, and
+// gradients that are not 16-byte aligned.  The one-hot positions are written
+// again after the row, each with the gradients of every id equal to its own.
+template <int NT, int NB>
+__global__ __launch_bounds__(NT) void k_lp_bwd_any(BwdArgs a) {
     const int64_t r = blockIdx.x;
-    const uint16_t* row = row_ptr(logits, r, T, stride_b, stride_t);
-    uint16_t* grow = grad + r * V;
-    const float g = ng[r], l = nl[r];
-    for (int64_t e = threadIdx.x; e < V; e += NT)
-        grow[e] = __bfloat16_as_ushort(__float2bfloat16(g * fast_exp2(fmaf(bf16_to_f32(row[e]), kLog2e, l))));
+    const uint16_t* row = row_ptr(a.logits, r, a.T, a.stride_b, a.stride_t);
+    uint16_t* grow = a.out + r * a.V;
+    const BwdRow<NB> w = bwd_row<NB>(a, r);
+    auto term = [&](int64_t e) { return w.ng * fast_exp2(fmaf(bf16_to_f32(row[e]), kLog2e, w.nl)); };
+    for (int64_t e = threadIdx.x; e < a.V; e += NT) {
+        const float q = term(e);
+        grow[e] = bf16_bits(NB == 0 && w.y[0] == e ? q + w.g[0] : q);
+    }
+    if constexpr (NB > 0) {
+        static_assert(NT >= kMaxIds, "one thread per id");
+        __shared__ int64_t s_y[kMaxIds];
+        __shared__ float s_g[kMaxIds];
+        const int j = threadIdx.x;
+        int64_t y = -1;
+        float g = 0.f;
+        if (j < a.n_ids) {
+            row_id(a, r, j, y, g);
+            s_y[j] = y;
+            s_g[j] = g;
+        }
+        __syncthreads();
+        if (y < 0) return;
+        float q = term(y);
+        for (int k = 0; k < a.n_ids; ++k) q += s_y[k] == y ? s_g[k] : 0.f;
+        grow[y] = bf16_bits(q);
+    }
 }
 
-// One thread per (row, id): the final value at the id's position, i.e. the
-// softmax term recomputed exactly as the streaming pass computed it, plus the
-// gradients of every id of the row equal to this one.  Threads of duplicate
-// ids store the same value.
-__global__ __launch_bounds__(256) void k_lp_bwd_fix(const uint16_t* __restrict__ logits, int64_t T, int64_t V,
-                                                    int64_t stride_b, int64_t stride_t,
-                                                    const int64_t* __restrict__ ids, int n_ids,
-                                                    const float* __restrict__ grad,
-                                                    const float* __restrict__ ng,
-                                                    const float* __restrict__ nl, int64_t n_rows,
-                                                    uint16_t* __restrict__ out) {
-    const int64_t j = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-    if (j >= n_rows * n_ids) return;
-    const int64_t r = j / n_ids;
-    const int64_t y = ids[j];
-    if (y < 0 || y >= V) return;  // ignored id, or a NaN row already written
-    const float g = ng[r];
-    if (isnan(g)) return;
-    const uint16_t* row = row_ptr(logits, r, T, stride_b, stride_t);
-    float q = g * fast_exp2(fmaf(bf16_to_f32(row[y]), kLog2e, nl[r]));
-    for (int k = 0; k < n_ids; ++k)
-        if (ids[r * n_ids + k] == y) q += grad[r * n_ids + k];
-    out[r * V + y] = __bfloat16_as_ushort(__float2bfloat16(q));
-}
-
-// 8 16-byte loads in flight per thread per tile (4 are slower at every size).
-// The flat backward: 256 threads x 4 loads, 65536 workgroups (sweep over
-// 16384..65536 workgroups, 2..8 loads).
+// 16-byte loads in flight per thread per tile (4 are slower at every size).
 constexpr int kFwdUnroll = 8;
 constexpr int kBwdThreads = 256;
-constexpr int kBwdUnroll = 4;
-constexpr uint32_t kBwdFlatBlocks = 65536;
-constexpr int kMaxIds = 256;  // gather ids per row (one thread each)
+constexpr int kBwdUnroll = 2;
+constexpr int64_t kBwdMinFlatV = 256;
+constexpr int64_t kBwdMaxElems = int64_t{1} << 33;  // of one launch: 32-bit chunk indices
 
 // Shape checks; an empty call (rows * T == 0) accepts NULL arrays, as an
 // empty tensor has no storage.
@@ -301,10 +418,6 @@ int check_common(const void* logits, int64_t rows, int64_t T, int64_t V, int64_t
     if (T > 0 && rows > INT32_MAX / T) return set_error(MESHY_EINVAL, "%s: too many rows", who);
     if (!logits && rows * T > 0) return set_error(MESHY_ENULL, "%s: logits is NULL", who);
     return MESHY_OK;
-}
-
-bool vector_ok(const void* logits, int64_t stride_b, int64_t stride_t) {
-    return (reinterpret_cast<uintptr_t>(logits) % 16 == 0) && (stride_b % 8 == 0) && (stride_t % 8 == 0);
 }
 
 // Threads of a row's workgroup.  Up to 256 rows there is one workgroup per CU
@@ -337,48 +450,67 @@ int launch_fwd(const uint16_t* logits, int64_t rows, int64_t T, int64_t V, int64
     return check_launch(who);
 }
 
+// The workspace that the backward's entry points have always asked for.  The
+// single pass needs none; they go on refusing a call without it.
 size_t bwd_ws_bytes(int64_t n_rows) { return 2 * align_up(sizeof(float) * static_cast<size_t>(n_rows), 256); }
+
+int check_bwd_ws(int64_t n, const void* workspace, size_t workspace_bytes, const char* who) {
+    if (!workspace || workspace_bytes < bwd_ws_bytes(n))
+        return set_error(MESHY_ESPACE, "%s: workspace needs %zu bytes", who, bwd_ws_bytes(n));
+    return MESHY_OK;
+}
 
 int launch_bwd(const uint16_t* logits, int64_t rows, int64_t T, int64_t V, int64_t stride_b,
                int64_t stride_t, const int64_t* ids, int n_ids, const float* lse, const float* grad_out,
-               uint16_t* grad_logits, void* workspace, size_t workspace_bytes, hipStream_t stream,
-               const char* who) {
+               uint16_t* grad_logits, hipStream_t stream, const char* who) {
     const int64_t n = rows * T;
-    if (n == 0) return MESHY_OK;
-    if (!workspace || workspace_bytes < bwd_ws_bytes(n))
-        return set_error(MESHY_ESPACE, "%s: workspace needs %zu bytes", who, bwd_ws_bytes(n));
-    float* ng = static_cast<float*>(workspace);
-    float* nl = reinterpret_cast<float*>(static_cast<char*>(workspace) + bwd_ws_bytes(n) / 2);
-    const unsigned row_blocks = static_cast<unsigned>(ceil_div(n, 256));
-    hipLaunchKernelGGL(k_lp_bwd_prep, dim3(row_blocks), dim3(256), 0, stream, ids, n_ids, lse, grad_out, n, V, ng,
-                       nl);
-    int rc = check_launch(who);
-    if (rc) return rc;
-    const bool vec = vector_ok(logits, stride_b, stride_t) && reinterpret_cast<uintptr_t>(grad_logits) % 16 == 0 &&
-                     V % 8 == 0;
-    const bool contiguous = stride_t == V && (rows == 1 || stride_b == T * V);
-    const int64_t n_chunks = n * (V / 8);
-    // The grid-stride index stays below 2^32: n_chunks plus one grid stride.
-    if (vec && contiguous && n_chunks <= (int64_t{1} << 32) - (int64_t{1} << 28)) {
-        const int64_t need = ceil_div(n_chunks, kBwdThreads * kBwdUnroll);
-        const unsigned blocks = static_cast<unsigned>(std::min<int64_t>(need, kBwdFlatBlocks));
-        hipLaunchKernelGGL((k_lp_bwd_flat<kBwdThreads, kBwdUnroll>), dim3(blocks), dim3(kBwdThreads), 0, stream,
-                           reinterpret_cast<const v4u*>(logits), static_cast<uint32_t>(V / 8),
-                           static_cast<uint32_t>(n_chunks), 1.0 / static_cast<double>(V / 8), ng, nl,
-                           reinterpret_cast<v4u*>(grad_logits));
-    } else if (vec) {
-        hipLaunchKernelGGL((k_lp_bwd_rows<kBwdThreads, kBwdUnroll>), dim3(static_cast<unsigned>(n)),
-                           dim3(kBwdThreads), 0, stream, logits, T, V, stride_b, stride_t, ng, nl, grad_logits);
+    BwdArgs a{};
+    a.logits = logits;
+    a.T = T, a.V = V, a.stride_b = stride_b, a.stride_t = stride_t;
+    a.inv_v = 1.0 / static_cast<double>(V);
+    a.ids = ids, a.lse = lse, a.grad_logp = grad_out;
+    a.out = grad_logits;
+    a.n_ids = n_ids;
+    // The ids that a lane holds, in blocks of 64.
+    auto by_ids = [&](auto go) {
+        if (n_ids == 1) go(std::integral_constant<int, 0>());
+        else if (n_ids <= kWave) go(std::integral_constant<int, 1>());
+        else if (n_ids <= 2 * kWave) go(std::integral_constant<int, 2>());
+        else go(std::integral_constant<int, kMaxIds / kWave>());
+    };
+    int rc;
+    const bool contiguous = stride_t == V && (rows == 1 || stride_b == T * V) &&
+                            reinterpret_cast<uintptr_t>(logits) % 16 == 0;
+    // A wave takes the rows that it holds in turn: at 2 rows per group of 512
+    // elements that is as fast as one workgroup per row with 2-byte accesses.
+    if (V >= kBwdMinFlatV && reinterpret_cast<uintptr_t>(grad_logits) % 16 == 0) {
+        const int64_t step = std::max<int64_t>(8, kBwdMaxElems / V / 8 * 8);
+        for (int64_t r0 = 0; r0 < n; r0 += step) {
+            a.row0 = r0;
+            a.n_elems = std::min(step, n - r0) * V;
+            a.n_chunks = static_cast<uint32_t>(ceil_div(a.n_elems, 8));
+            const dim3 blocks(static_cast<unsigned>(ceil_div(a.n_chunks, kBwdThreads * kBwdUnroll)));
+            by_ids([&](auto nb) {
+                constexpr int NB = decltype(nb)::value;
+                if (contiguous)
+                    hipLaunchKernelGGL((k_lp_bwd_flat<kBwdThreads, kBwdUnroll, NB, true>), blocks, dim3(kBwdThreads),
+                                       0, stream, a);
+                else
+                    hipLaunchKernelGGL((k_lp_bwd_flat<kBwdThreads, kBwdUnroll, NB, false>), blocks, dim3(kBwdThreads),
+                                       0, stream, a);
+            });
+            if ((rc = check_launch(who))) return rc;
+            a.ids += step * n_ids, a.lse += step, a.grad_logp += step * n_ids, a.out += step * V;
+        }
     } else {
-        hipLaunchKernelGGL((k_lp_bwd_any<kBwdThreads>), dim3(static_cast<unsigned>(n)), dim3(kBwdThreads), 0,
-                           stream, logits, T, V, stride_b, stride_t, ng, nl, grad_logits);
+        const dim3 blocks(static_cast<unsigned>(n));
+        by_ids([&](auto nb) {
+            hipLaunchKernelGGL((k_lp_bwd_any<kBwdThreads, decltype(nb)::value>), blocks, dim3(kBwdThreads), 0, stream,
+                               a);
+        });
+        return check_launch(who);
     }
-    rc = check_launch(who);
-    if (rc) return rc;
-    const unsigned fix_blocks = static_cast<unsigned>(ceil_div(n * n_ids, 256));
-    hipLaunchKernelGGL(k_lp_bwd_fix, dim3(fix_blocks), dim3(256), 0, stream, logits, T, V, stride_b, stride_t, ids,
-                       n_ids, grad_out, ng, nl, n, grad_logits);
-    return check_launch(who);
+    return MESHY_OK;
 }
 
 }  // namespace
@@ -432,57 +564,12 @@ extern "C" int meshy_logprob_bwd(const uint16_t* logits, int64_t rows, int64_t T
     if (rows * T == 0) return MESHY_OK;
     if (!labels || !lse || !grad_logp || !grad_logits)
         return set_error(MESHY_ENULL, "%s: labels, lse, grad_logp and grad_logits are required", who);
-    return launch_bwd(logits, rows, T, V, stride_b, stride_t, labels, 1, lse, grad_logp, grad_logits, workspace,
-                      workspace_bytes, stream, who);
+    if ((rc = check_bwd_ws(rows * T, workspace, workspace_bytes, who))) return rc;
+    return launch_bwd(logits, rows, T, V, stride_b, stride_t, labels, 1, lse, grad_logp, grad_logits, stream, who);
 }
 
-// ------------------------------------------------ allocation-free backward
-//
-// meshy_logprob_bwd_noalloc runs the kernels of meshy_logprob_bwd with their
-// two floats per row (-G and -lse log2 e) in this file-scope device array
-// instead of a caller workspace.  Each GPU holds its own copy; host code
-// reaches it only through the address hipGetSymbolAddress reports for the
-// current device, looked up once per device and cached below.  Nothing in it
-// must start at zero: the prep kernel writes every row's pair before the
-// streaming pass and the fixup read it.  Calls that overlap on one GPU (on
-// different streams) share the array and race.
-static __device__ __align__(256) float scratch[2 * MESHY_NOALLOC_MAX_ROWS];
-
-namespace meshy {
-namespace {
-
-constexpr int kMaxDevices = 64;
-std::atomic<float*> g_scratch[kMaxDevices];
-std::mutex g_scratch_mu;
-
-// The current device's copy of `scratch` (looked up on its first use).
-int scratch_of_current_device(float** out, const char* who) {
-    int dev = -1;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return set_error(static_cast<int>(e), "%s: hipGetDevice: %s", who, hipGetErrorString(e));
-    if (dev < 0 || dev >= kMaxDevices) return set_error(MESHY_EINVAL, "%s: device %d out of range", who, dev);
-    float* p = g_scratch[dev].load(std::memory_order_acquire);
-    if (!p) {
-        std::lock_guard<std::mutex> lock(g_scratch_mu);
-        p = g_scratch[dev].load(std::memory_order_relaxed);
-        if (!p) {
-            void* addr = nullptr;
-            e = hipGetSymbolAddress(&addr, HIP_SYMBOL(scratch));
-            if (e != hipSuccess || !addr)
-                return set_error(e != hipSuccess ? static_cast<int>(e) : MESHY_EINVAL,
-                                 "%s: hipGetSymbolAddress(scratch) on device %d: %s", who, dev,
-                                 hipGetErrorString(e));
-            p = static_cast<float*>(addr);
-            g_scratch[dev].store(p, std::memory_order_release);
-        }
-    }
-    *out = p;
-    return MESHY_OK;
-}
-
-}  // namespace
-}  // namespace meshy
-
+// meshy_logprob_bwd without the workspace argument, for callers that cannot
+// allocate; it keeps the row limit that it is declared with.
 extern "C" int meshy_logprob_bwd_noalloc(const uint16_t* logits, int64_t rows, int64_t T, int64_t V,
                                          int64_t stride_b, int64_t stride_t, const int64_t* labels,
                                          const float* lse, const float* grad_logp, uint16_t* grad_logits,
@@ -497,13 +584,9 @@ extern "C" int meshy_logprob_bwd_noalloc(const uint16_t* logits, int64_t rows, i
     if (!labels || !lse || !grad_logp || !grad_logits)
         return set_error(MESHY_ENULL, "%s: labels, lse, grad_logp and grad_logits are required", who);
     if (n > MESHY_NOALLOC_MAX_ROWS)
-        return set_error(MESHY_ESPACE, "%s: %lld rows exceed the static scratch of %d rows", who,
+        return set_error(MESHY_ESPACE, "%s: %lld rows exceed the static scratch limit of %d rows", who,
                          static_cast<long long>(n), MESHY_NOALLOC_MAX_ROWS);
-    float* ws = nullptr;
-    rc = scratch_of_current_device(&ws, who);
-    if (rc) return rc;
-    return launch_bwd(logits, rows, T, V, stride_b, stride_t, labels, 1, lse, grad_logp, grad_logits, ws,
-                      bwd_ws_bytes(n), stream, who);
+    return launch_bwd(logits, rows, T, V, stride_b, stride_t, labels, 1, lse, grad_logp, grad_logits, stream, who);
 }
 
 extern "C" int meshy_gather_logprobs_bwd(const uint16_t* logits, int64_t rows, int64_t T, int64_t V,
@@ -522,8 +605,9 @@ extern "C" int meshy_gather_logprobs_bwd(const uint16_t* logits, int64_t rows, i
     if (rows * T == 0) return MESHY_OK;
     if (!ids || !lse || !grad_out || !grad_logits)
         return set_error(MESHY_ENULL, "%s: ids, lse, grad_out and grad_logits are required", who);
+    if ((rc = check_bwd_ws(rows * T, workspace, workspace_bytes, who))) return rc;
     return launch_bwd(logits, rows, T, V, stride_b, stride_t, ids, static_cast<int>(n_ids), lse, grad_out,
-                      grad_logits, workspace, workspace_bytes, stream, who);
+                      grad_logits, stream, who);
 }
 
 namespace meshy {
