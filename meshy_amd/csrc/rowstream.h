@@ -26,14 +26,15 @@ constexpr int64_t kIgnoreIndex = -100;
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
-// Merges (m2, s2, t2) into (m, s, t).
+// Merges (m2, s2, t2) into (m, s, t); kEntropy = false leaves t untouched.
+template <bool kEntropy = true>
 __device__ __forceinline__ void merge(float& m, float& s, float& t, float m2, float s2, float t2) {
     const float mn = fmaxf(m, m2);
     const float d1 = (m - mn) * kLog2e;
     const float d2 = (m2 - mn) * kLog2e;
     const float a1 = fast_exp2(d1);
     const float a2 = fast_exp2(d2);
-    t = a1 * fmaf(d1, s, t) + a2 * fmaf(d2, s2, t2);
+    if (kEntropy) t = a1 * fmaf(d1, s, t) + a2 * fmaf(d2, s2, t2);
     s = a1 * s + a2 * s2;
     m = mn;
 }
@@ -188,41 +189,42 @@ __device__ __forceinline__ void accumulate_one(float z, bool ok, float& m, float
 }
 
 // Merges each lane's triple with that of the lane kCtrl rotates to it.
-template <int kCtrl>
+template <int kCtrl, bool kEntropy>
 __device__ __forceinline__ void merge_dpp(float& m, float& s, float& t) {
     const float m2 = dpp_f32<kCtrl>(m);
     const float s2 = dpp_f32<kCtrl>(s);
-    const float t2 = dpp_f32<kCtrl>(t);
-    merge(m, s, t, m2, s2, t2);
+    const float t2 = kEntropy ? dpp_f32<kCtrl>(t) : 0.f;
+    merge<kEntropy>(m, s, t, m2, s2, t2);
 }
 
 // The merge over each 16-lane row through DPP rotations, valid in lane 0 of
 // the row.
+template <bool kEntropy>
 __device__ __forceinline__ void merge_rows16(float& m, float& s, float& t) {
-    merge_dpp<kDppRowRor8>(m, s, t);
-    merge_dpp<kDppRowRor4>(m, s, t);
-    merge_dpp<kDppRowRor2>(m, s, t);
-    merge_dpp<kDppRowRor1>(m, s, t);
+    merge_dpp<kDppRowRor8, kEntropy>(m, s, t);
+    merge_dpp<kDppRowRor4, kEntropy>(m, s, t);
+    merge_dpp<kDppRowRor2, kEntropy>(m, s, t);
+    merge_dpp<kDppRowRor1, kEntropy>(m, s, t);
 }
 
 // Block-wide merge of the per-lane triples; the result lands in thread 0.
 // Rows of 16 lanes and then the waves' triples go through DPP rotations: with
 // 16 waves a chain of one merge per wave in thread 0 alone took longer than
 // the rest of the merge.
-template <int NT>
+template <int NT, bool kEntropy = true>
 __device__ __forceinline__ void block_merge(float& m, float& s, float& t) {
-    merge_rows16(m, s, t);
+    merge_rows16<kEntropy>(m, s, t);
     float mr[4], sr[4], tr[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         mr[r] = lane_f32(m, 16 * r);
         sr[r] = lane_f32(s, 16 * r);
-        tr[r] = lane_f32(t, 16 * r);
+        tr[r] = kEntropy ? lane_f32(t, 16 * r) : 0.f;
     }
-    merge(mr[0], sr[0], tr[0], mr[1], sr[1], tr[1]);
-    merge(mr[2], sr[2], tr[2], mr[3], sr[3], tr[3]);
+    merge<kEntropy>(mr[0], sr[0], tr[0], mr[1], sr[1], tr[1]);
+    merge<kEntropy>(mr[2], sr[2], tr[2], mr[3], sr[3], tr[3]);
     m = mr[0], s = sr[0], t = tr[0];
-    merge(m, s, t, mr[2], sr[2], tr[2]);
+    merge<kEntropy>(m, s, t, mr[2], sr[2], tr[2]);
     if constexpr (NT > kWave) {
         constexpr int kWaves = NT / kWave;
         static_assert(kWaves <= 16, "the waves' triples are merged in one row of 16 lanes");
@@ -232,15 +234,15 @@ __device__ __forceinline__ void block_merge(float& m, float& s, float& t) {
         if (lane == 0) {
             sm[wid] = m;
             ss[wid] = s;
-            st[wid] = t;
+            if (kEntropy) st[wid] = t;
         }
         __syncthreads();
         if (wid == 0) {
             const bool in = lane < kWaves;
             m = in ? sm[lane] : kInit;
             s = in ? ss[lane] : 0.f;
-            t = in ? st[lane] : 0.f;
-            merge_rows16(m, s, t);
+            t = kEntropy && in ? st[lane] : 0.f;
+            merge_rows16<kEntropy>(m, s, t);
         }
     }
 }
@@ -254,15 +256,16 @@ constexpr int kLineElems = 64;  // elements of a 128-byte line
 struct RowSpan {
     const v4u* body;
     int64_t n8;
-    int head;  // < kLineElems
+    int line;  // elements from the row's start to the boundary (< kLineElems)
+    int head;  // line, or V if the row ends before it
     int tail;  // < 8
 };
 
 __device__ __forceinline__ RowSpan row_span(const uint16_t* row, int64_t V) {
     RowSpan sp;
     const uintptr_t past = reinterpret_cast<uintptr_t>(row) % (2 * kLineElems);
-    const int64_t to_line = past ? static_cast<int64_t>((2 * kLineElems - past) / 2) : 0;
-    sp.head = static_cast<int>(min(to_line, V));
+    sp.line = past ? static_cast<int>((2 * kLineElems - past) / 2) : 0;
+    sp.head = static_cast<int>(min(static_cast<int64_t>(sp.line), V));
     sp.body = reinterpret_cast<const v4u*>(row + sp.head);
     sp.n8 = (V - sp.head) >> 3;
     sp.tail = static_cast<int>((V - sp.head) & 7);
