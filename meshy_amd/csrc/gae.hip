@@ -502,25 +502,44 @@ __global__ __launch_bounds__(kCountThreads) void k_gae_count(meshy_gae_args g, f
 }
 
 // Masked token count of document blockIdx.x over its offsets range: every
-// thread sums a fixed set of positions (four loads in flight), then a
-// fixed-order block sum; the result does not depend on timing.
-__global__ __launch_bounds__(kCountThreads) void k_gae_doc_count(const float* __restrict__ mask,
-                                                                 const int64_t* __restrict__ off,
-                                                                 float* __restrict__ cnt) {
-    __shared__ float s_red[kCountThreads / kWave];
+// thread sums a fixed set of positions, then a fixed-order block sum; the
+// result does not depend on timing.  Bound by the longest documents, one
+// workgroup each: 16 positions per thread and step, in four 16-byte loads in
+// flight together (vec: the mask is 16-byte aligned), take 6.0 us for the 1024
+// documents of 6.35 M tokens, 12.3 with four 4-byte loads and 256 threads.
+constexpr int kDocCountThreads = 512;
+
+__global__ __launch_bounds__(kDocCountThreads) void k_gae_doc_count(const float* __restrict__ mask,
+                                                                    const int64_t* __restrict__ off, bool vec,
+                                                                    float* __restrict__ cnt) {
+    __shared__ float s_red[kDocCountThreads / kWave];
     const int64_t d = blockIdx.x;
     const int64_t lo = off[d];
     const int64_t hi = off[d + 1];
+    const int tid = threadIdx.x;
+    // Groups of four positions [4 g0, 4 g1), and what lies before and after.
+    const int64_t g0 = vec ? (lo + 3) / 4 : hi;
+    const int64_t g1 = vec ? max(hi / 4, g0) : g0;
+    const int64_t head = vec ? min(4 * g0, hi) : hi;
     float acc = 0.f;
-    int64_t t = lo + threadIdx.x;
-    for (; t + 3 * kCountThreads < hi; t += 4 * kCountThreads) {
-        const float a0 = mask[t], a1 = mask[t + kCountThreads], a2 = mask[t + 2 * kCountThreads],
-                    a3 = mask[t + 3 * kCountThreads];
-        acc += (a0 + a1) + (a2 + a3);
+    constexpr int kIn = 4;
+    for (int64_t g = g0 + tid; g < g1; g += kIn * kDocCountThreads) {
+        f32x4 m[kIn];
+#pragma unroll
+        for (int u = 0; u < kIn; ++u)
+            m[u] = *reinterpret_cast<const f32x4*>(mask + 4 * min(g + u * kDocCountThreads, g1 - 1));
+#pragma unroll
+        for (int u = 0; u < kIn; ++u) {
+            const float s = (m[u].x + m[u].y) + (m[u].z + m[u].w);
+            acc += g + u * kDocCountThreads < g1 ? s : 0.f;
+        }
     }
-    for (; t < hi; t += kCountThreads) acc += mask[t];
-    acc = block_sum<kCountThreads>(acc, s_red);
-    if (threadIdx.x == 0) cnt[d] = acc;
+    for (int64_t t = lo + tid; t < head; t += kDocCountThreads) acc += mask[t];
+    if (vec) {
+        for (int64_t t = max(4 * g1, head) + tid; t < hi; t += kDocCountThreads) acc += mask[t];
+    }
+    acc = block_sum<kDocCountThreads>(acc, s_red);
+    if (tid == 0) cnt[d] = acc;
 }
 
 // The thread's maps (contiguous positions) folded right to left.
@@ -933,8 +952,8 @@ int gae_launch(const meshy_gae_args& g, hipStream_t stream) {
     // Document lengths only matter for lambda (advantages / lam_doc), not for returns.
     if (!g.lengths && (g.adv || g.lam_doc) && g.seg_offsets) {
         if (g.n_docs > 0) {
-            hipLaunchKernelGGL(k_gae_doc_count, dim3(static_cast<unsigned>(g.n_docs)), dim3(kCountThreads), 0,
-                               stream, g.mask, g.seg_offsets, ws.cnt);
+            hipLaunchKernelGGL(k_gae_doc_count, dim3(static_cast<unsigned>(g.n_docs)), dim3(kDocCountThreads), 0,
+                               stream, g.mask, g.seg_offsets, reinterpret_cast<uintptr_t>(g.mask) % 16 == 0, ws.cnt);
             if ((rc = check_launch("meshy_gae(count)"))) return rc;
         }
     } else if (!g.lengths && (g.adv || g.lam_doc)) {
