@@ -505,8 +505,8 @@ __global__ __launch_bounds__(kCountThreads) void k_gae_count(meshy_gae_args g, f
 // thread sums a fixed set of positions, then a fixed-order block sum; the
 // result does not depend on timing.  Bound by the longest documents, one
 // workgroup each: 16 positions per thread and step, in four 16-byte loads in
-// flight together (vec: the mask is 16-byte aligned), take 6.0 us for the 1024
-// documents of 6.35 M tokens, 12.3 with four 4-byte loads and 256 threads.
+// flight together (vec: the mask is 16-byte aligned), take 7.0 us for the 1024
+// documents of 6.35 M tokens, 11.9 with four 4-byte loads and 256 threads.
 constexpr int kDocCountThreads = 512;
 
 __global__ __launch_bounds__(kDocCountThreads) void k_gae_doc_count(const float* __restrict__ mask,
@@ -563,16 +563,14 @@ __device__ __forceinline__ Pair chunk_map(const Pair (&items)[kItems], Pair* s_w
     return total;
 }
 
-// The chunk's map for the slots.  A plain fold is NaN or infinite exactly
-// when one of its terms is (0 * NaN, 0 * inf and NaN + x are all NaN), so the
-// plain map tells whether the chunk holds a non-finite term; only then is the
-// map composed again with hardness.  A plain map takes its hardness (a row end
-// in the chunk) from the positions.  Every thread returns the same map.
-__device__ __forceinline__ Pair published_map(const Pair (&items)[kItems], bool has_row_end, Pair* s_wave,
-                                              Pair* s_wave_hard, int* s_row_end, bool& nonfinite) {
-    const bool wave_row_end = __ballot(has_row_end) != 0;
-    if (threadIdx.x % kWave == 0) s_row_end[threadIdx.x / kWave] = wave_row_end;
-    Pair total = chunk_map<false>(items, s_wave);  // its barrier publishes s_row_end
+// The chunk's map for the slots, from the plain composition of its maps
+// (`total`).  A plain fold is NaN or infinite exactly when one of its terms is
+// (0 * NaN, 0 * inf and NaN + x are all NaN), so it tells whether the chunk
+// holds a non-finite term; only then is the map composed again with hardness.
+// A plain map takes its hardness (a row end in the chunk, s_row_end) from the
+// positions.  Every thread returns the same map.
+__device__ __forceinline__ Pair published_map(const Pair (&items)[kItems], Pair total, const int* s_row_end,
+                                              Pair* s_wave_hard, bool& nonfinite) {
     nonfinite = !isfinite(total.adv.q) || !isfinite(total.ret.q);
     if (nonfinite) return chunk_map<true>(items, s_wave_hard);
     bool hard = false;
@@ -594,17 +592,13 @@ __global__ __launch_bounds__(kThreads) void k_gae_lambda(meshy_gae_args g, const
                  static_cast<int64_t>(gridDim.x) * kThreads);
 }
 
-// The chunk's outputs from its carry-in (s_carry, written by wave 0 before
-// the call): scans the threads from the right seeded with the carry and
-// writes A_t and G_t.
+// The chunk's outputs from its carry-in: A_t and G_t of the thread's
+// positions, scanned from the right (excl: the map of the threads after it).
 template <bool kHard>
-__device__ __forceinline__ void scan_and_write(const meshy_gae_args& g, int64_t n, bool vec, int64_t c,
-                                               Pair* s_suffix, const float* s_carry, const Pair (&items)[kItems],
-                                               uint32_t valid_bits) {
+__device__ __forceinline__ void write_outputs(const meshy_gae_args& g, int64_t n, bool vec, int64_t c, const Pair& excl,
+                                              const float* s_carry, const Pair (&items)[kItems],
+                                              uint32_t valid_bits) {
     const int64_t t0 = c * kChunk + static_cast<int64_t>(threadIdx.x) * kItems;
-    const Pair mine = fold_items<kHard>(items);
-    Pair total;
-    const Pair excl = block_suffix_exclusive<kHard>(mine, s_suffix, total);  // its barriers publish s_carry
     float A = apply_map<kHard>(excl.adv, s_carry[0]);
     float G = apply_map<kHard>(excl.ret, s_carry[1]);
     float outA[kItems], outG[kItems];
@@ -667,9 +661,6 @@ constexpr int kFirstBatch = 4;
 // redoes the call's outputs.
 __global__ __launch_bounds__(kThreads) void k_gae_scan(meshy_gae_args g, Workspace ws, int64_t n, int64_t nc,
                                                        bool vec, unsigned long long epoch, int max_polls) {
-    // The chunk map and the suffix scan use separate arrays: a wave may enter
-    // the scan while another still reads the map's array.
-    __shared__ Pair s_wave[kThreads / kWave];
     __shared__ Pair s_wave_hard[kThreads / kWave];
     __shared__ Pair s_suffix[kThreads / kWave];
     __shared__ int s_row_end[kThreads / kWave];
@@ -681,8 +672,15 @@ __global__ __launch_bounds__(kThreads) void k_gae_scan(meshy_gae_args g, Workspa
     bool has_row_end;
     thread_maps(g, ws.cnt, c * kChunk, c * kChunk + static_cast<int64_t>(threadIdx.x) * kItems, n, vec, items,
                 valid_bits, has_row_end);
+    // One scan gives the chunk's map and each thread's suffix: only the carry is
+    // left to apply once the neighbours' maps have come (27.8 us against 28.6
+    // with a fold for the map first and the scan after the wait).
+    const bool wave_row_end = __ballot(has_row_end) != 0;
+    if (lane == 0) s_row_end[threadIdx.x / kWave] = wave_row_end;
+    Pair total;
+    const Pair excl = block_suffix_exclusive<false>(fold_items<false>(items), s_suffix, total);
     bool nonfinite;
-    const Pair total = published_map(items, has_row_end, s_wave, s_wave_hard, s_row_end, nonfinite);
+    total = published_map(items, total, s_row_end, s_wave_hard, nonfinite);
     if (threadIdx.x < 4) {
         const float v = threadIdx.x == 0 ? total.adv.p
                         : threadIdx.x == 1 ? total.adv.q
@@ -727,7 +725,8 @@ __global__ __launch_bounds__(kThreads) void k_gae_scan(meshy_gae_args g, Workspa
             s_carry[1] = carry.ret.q;
         }
     }
-    scan_and_write<false>(g, n, vec, c, s_suffix, s_carry, items, valid_bits);
+    __syncthreads();
+    write_outputs<false>(g, n, vec, c, excl, s_carry, items, valid_bits);
     if (g.lam_doc) write_lambda(g, ws.cnt, static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x,
                                 static_cast<int64_t>(gridDim.x) * kThreads);
 }
@@ -768,7 +767,9 @@ __global__ __launch_bounds__(kThreads) void k_gae_fix(meshy_gae_args g, Workspac
                 s_carry[1] = carry.ret.q;
             }
         }
-        scan_and_write<true>(g, n, vec, c, s_wave, s_carry, items, valid_bits);
+        Pair total;
+        const Pair excl = block_suffix_exclusive<true>(fold_items<true>(items), s_wave, total);  // publishes s_carry
+        write_outputs<true>(g, n, vec, c, excl, s_carry, items, valid_bits);
         __syncthreads();  // s_carry is read after the scan's last barrier
     }
 }
