@@ -836,20 +836,17 @@ class _PackViews:
         return self.seg[d0:d0 + nd + 2]
 
     # Each group's views are made for every micro at once, the first time any
-    # micro needs them: one torch.split per tensor (a third of a microsecond
-    # per view) instead of a slice and a view per micro and field.
+    # micro needs them: the per-token tensors by one native call, the others by
+    # one torch.split per tensor (a third of a microsecond per view) instead of
+    # a slice and a view per micro and field.
 
     def _token_views(self) -> list:
         if self._tok is None:
-            sizes = self.sizes
-            tok = [self._flat(name) for name in self._TOK]
-            if self.packed:
-                cols = [None if t is None else torch.split(t.view(1, -1), sizes, dim=1) for t in tok]
-            else:
-                cols = [None if t is None else [p.view(R, S) for p, R, S in zip(torch.split(t, sizes), self.rows,
-                                                                                 self.seq)]
-                        for t in tok]
-            self._tok = [tuple(None if c is None else c[k] for c in cols) for k in range(len(sizes))]
+            regions = self.out_lay.regions
+            specs = tuple((regions[name][0], _SCALAR_TYPE[regions[name][2]]) if name in regions else None
+                          for name in self._TOK)
+            rows, seq = (np.asarray(x, np.int64).tobytes() for x in (self._job.rows, self._job.seq))
+            self._tok = _lib.stage().token_views(self.obuf, specs, rows, seq)
         return self._tok
 
     def tokens(self, mb: "PackedBatch", f: dict) -> None:

@@ -53,8 +53,16 @@
 //       for an absent region), the four tables as bytes, and the compact
 //       sample map with each used sample's prefix length as plan_tables
 //       gives them.
+//   token_views(buf, regions, rows, seq)
+//       The per-token tensors of every micro of a pack launch: regions is one
+//       (byte offset in buf, c10::ScalarType) or None per output, rows and seq
+//       the micros' shapes as int64 bytes; returns one tuple per micro of its
+//       [rows, seq] tensors (None for an absent output).  A micro's elements
+//       follow the previous micro's in each region.  The tensors share buf's
+//       storage and version counter, as buf[a:b].view(dtype) would.
 #include <Python.h>
 
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <algorithm>
@@ -670,12 +678,99 @@ PyObject* stage_micros(PyObject*, PyObject* args) {
                          to_bytes(doc_start), to_bytes(used), to_bytes(need));
 }
 
+// A [rows, seq] tensor of `type` over buf's storage from element `offset`.
+at::Tensor typed_view(const at::Tensor& buf, caffe2::TypeMeta type, int64_t offset, int64_t rows, int64_t seq) {
+    auto impl = c10::make_intrusive<c10::TensorImpl>(c10::Storage(buf.storage()), buf.key_set(), type);
+    impl->set_storage_offset(offset);
+    impl->set_sizes_contiguous({rows, seq});
+    impl->set_version_counter(buf.unsafeGetTensorImpl()->version_counter());
+    return at::Tensor(std::move(impl));
+}
+
+// Slicing, splitting and viewing each output through torch's Python API took
+// about half of a pack step of 7 micros whose 42 tensors are read: the step
+// takes 101 us with it and 55 with this pass.
+PyObject* token_views(PyObject*, PyObject* args) {
+    HANDLE_TH_ERRORS
+    PyObject *py_buf, *py_regions, *py_rows, *py_seq;
+    if (!PyArg_ParseTuple(args, "OO!O!O!", &py_buf, &PyTuple_Type, &py_regions, &PyBytes_Type, &py_rows,
+                          &PyBytes_Type, &py_seq))
+        return nullptr;
+    if (!THPVariable_Check(py_buf)) {
+        PyErr_SetString(PyExc_TypeError, "token_views: buf must be a tensor");
+        return nullptr;
+    }
+    const at::Tensor& buf = THPVariable_Unpack(py_buf);
+    const Py_ssize_t n_micro = PyBytes_GET_SIZE(py_seq) / static_cast<Py_ssize_t>(sizeof(int64_t));
+    const int64_t* rows = reinterpret_cast<const int64_t*>(PyBytes_AS_STRING(py_rows));
+    const int64_t* seq = reinterpret_cast<const int64_t*>(PyBytes_AS_STRING(py_seq));
+    TORCH_CHECK_VALUE(buf.scalar_type() == at::kByte && buf.is_contiguous(),
+                      "token_views: buf must be a contiguous uint8 tensor");
+    TORCH_CHECK_VALUE(PyBytes_GET_SIZE(py_rows) == PyBytes_GET_SIZE(py_seq), "token_views: rows and seq differ in length");
+    int64_t total = 0;
+    for (Py_ssize_t k = 0; k < n_micro; ++k) {
+        TORCH_CHECK_VALUE(rows[k] >= 0 && seq[k] >= 0, "token_views: negative sizes");
+        total += rows[k] * seq[k];
+    }
+    const Py_ssize_t n_out = PyTuple_GET_SIZE(py_regions);
+    struct Region {
+        caffe2::TypeMeta type;
+        int64_t at = -1;  // first element, -1 for an absent output
+    };
+    std::vector<Region> regions(static_cast<size_t>(n_out));
+    for (Py_ssize_t i = 0; i < n_out; ++i) {
+        PyObject* r = PyTuple_GET_ITEM(py_regions, i);
+        if (r == Py_None) continue;
+        long long byte;
+        int type;
+        if (!PyTuple_Check(r) || !PyArg_ParseTuple(r, "Li", &byte, &type)) {
+            if (!PyErr_Occurred()) PyErr_SetString(PyExc_TypeError, "token_views: a region is (offset, type) or None");
+            return nullptr;
+        }
+        TORCH_CHECK_VALUE(type >= 0 && type < static_cast<int>(at::ScalarType::NumOptions), "token_views: bad type");
+        const auto meta = c10::scalarTypeToTypeMeta(static_cast<at::ScalarType>(type));
+        const int64_t size = static_cast<int64_t>(meta.itemsize());
+        const int64_t first = buf.storage_offset() + byte;
+        TORCH_CHECK_VALUE(byte >= 0 && size > 0 && byte + total * size <= buf.numel() && first % size == 0,
+                          "token_views: a region lies outside the buffer or is not aligned");
+        regions[i] = Region{meta, first / size};
+    }
+    PyObject* out = PyList_New(n_micro);
+    if (!out) return nullptr;
+    int64_t at = 0;
+    for (Py_ssize_t k = 0; k < n_micro; ++k) {
+        PyObject* t = PyTuple_New(n_out);
+        if (!t) {
+            Py_DECREF(out);
+            return nullptr;
+        }
+        PyList_SET_ITEM(out, k, t);  // `out` owns it from here
+        for (Py_ssize_t i = 0; i < n_out; ++i) {
+            PyObject* v = Py_None;
+            if (regions[i].at < 0) {
+                Py_INCREF(v);
+            } else {
+                v = THPVariable_Wrap(typed_view(buf, regions[i].type, regions[i].at + at, rows[k], seq[k]));
+                if (!v) {
+                    Py_DECREF(out);
+                    return nullptr;
+                }
+            }
+            PyTuple_SET_ITEM(t, i, v);
+        }
+        at += rows[k] * seq[k];
+    }
+    return out;
+    END_HANDLE_TH_ERRORS
+}
+
 PyMethodDef kMethods[] = {
     {"gather", gather, METH_VARARGS, "Concatenate one column of the used samples into a host buffer."},
     {"plan_tables", plan_tables, METH_VARARGS, "Compact sample map and document tables of a list of micros."},
     {"columns", columns, METH_VARARGS, "Pointer, shape and dtype records of one column of the used samples."},
     {"scalars", scalars, METH_VARARGS, "One scalar field of the used samples as float64."},
     {"stage_micros", stage_micros, METH_VARARGS, "The whole staging of a list of micros, for the common case."},
+    {"token_views", token_views, METH_VARARGS, "The per-token tensors of every micro of a pack launch."},
     {nullptr, nullptr, 0, nullptr},
 };
 
