@@ -302,6 +302,14 @@ int meshy_zero_variance_groups_host(const double* raw_rewards, int64_t n_rewards
 int meshy_logprob_entropy_fwd(const uint16_t* logits, int64_t rows, int64_t T, int64_t V,
                               int64_t stride_b, int64_t stride_t, const int64_t* labels,
                               float* logp, float* entropy, float* lse, hipStream_t stream);
+/* Test hook, no counterpart in the reference: the same call, in which a
+ * workgroup that waits for the other parts of its row (few rows are divided
+ * over several workgroups) polls max_polls times (0 to the default of 4000)
+ * before it streams the whole row itself. */
+int meshy_logprob_entropy_fwd_polls(const uint16_t* logits, int64_t rows, int64_t T, int64_t V,
+                                    int64_t stride_b, int64_t stride_t, const int64_t* labels,
+                                    float* logp, float* entropy, float* lse, int32_t max_polls,
+                                    hipStream_t stream);
 
 /*
  * Backward of logp with respect to the logits:

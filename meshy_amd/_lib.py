@@ -276,6 +276,11 @@ SIGNATURES = {
         [c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64, c_void_p, c_void_p, c_void_p,
          c_void_p, c_void_p],
     ),
+    "meshy_logprob_entropy_fwd_polls": (
+        c_int,
+        [c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64, c_void_p, c_void_p, c_void_p,
+         c_void_p, c_int32, c_void_p],
+    ),
     "meshy_logprob_bwd_workspace_size": (c_size_t, [c_int64]),
     "meshy_logprob_bwd": (
         c_int,

@@ -18,6 +18,7 @@
 // [rows * V] gradient with a grid-stride loop: on MI355X that order writes 8 %
 // faster than one workgroup per row.
 #include <algorithm>
+#include <atomic>
 #include <type_traits>
 
 #include "rowstream.h"
@@ -92,20 +93,94 @@ __device__ __forceinline__ void accumulate_exact(v4u (&v)[U], float& m, float& s
     accumulate(z, m, s, t);
 }
 
-// Bound by the read of the logits.  NT threads per row (fwd_threads), U 16-byte
-// loads in flight per thread per tile.  A lane's first tile sets its running max; later tiles are accumulated against it
-// (accumulate_at) and take the tile max only when an element lies more than 44
-// above it.  The chunks left after the full tiles form one predicated tile.
+// A row's parts meet in slots: the triple of one part, each float in the low
+// half of a 64-bit word whose high half is a tag drawn from the call, the slot
+// and the word.  A word is one single-copy atomic, so a reader takes it exactly
+// when its tag is the call's; whatever else the slot held carries another tag,
+// and nothing is cleared.  Call e uses entry e % kSplitRing: a call overlapped
+// by a later one of the same entry (kSplitRing calls on, on another stream) can
+// lose a word, and then streams the whole row itself.
+constexpr int kMaxParts = 16;     // merged in one row of 16 lanes
+constexpr int kSplitSlots = 256;  // at least a launch's rows * parts
+constexpr int kSplitRing = 64;
+constexpr int kSplitPolls = 4000;  // of a waiting wave, some ms in all
+
+struct SplitSlot {
+    unsigned long long w[4];
+};
+__device__ SplitSlot g_split[kSplitRing][kSplitSlots];
+
+__device__ __forceinline__ uint32_t split_tag(unsigned long long call, int slot, int w) {
+    unsigned long long x = call * 0x9E3779B97F4A7C15ull + static_cast<unsigned>(slot * 4 + w) * 0xBF58476D1CE4E5B9ull;
+    x ^= x >> 31;
+    x *= 0x94D049BB133111EBull;
+    x ^= x >> 29;
+    return static_cast<uint32_t>(x >> 32);
+}
+
+// A split row's part merged with the others (wave 0 holds this part's triple in
+// lane 0): polls for the triples of parts 0 .. parts - 2 of row r and merges in
+// a fixed order, the result in lane 0.  Returns whether the polls ran out first.
+__device__ __forceinline__ bool merge_parts(const SplitSlot* slots, int r, int n_rows, int parts,
+                                            unsigned long long call, int max_polls, float& m, float& s, float& t) {
+    const int lane = threadIdx.x;
+    const bool own = lane + 1 == parts;
+    const float m0 = lane_f32(m, 0), s0 = lane_f32(s, 0), t0 = lane_f32(t, 0);
+    m = own ? m0 : kInit, s = own ? s0 : 0.f, t = own ? t0 : 0.f;
+    const int slot = lane * n_rows + r;
+    bool ready = lane + 1 >= parts;
+    for (int poll = 0;; ++poll) {
+        if (!ready) {
+            unsigned long long x[3];
+#pragma unroll
+            for (int w = 0; w < 3; ++w)
+                x[w] = __hip_atomic_load(&slots[slot].w[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            ready = static_cast<uint32_t>(x[0] >> 32) == split_tag(call, slot, 0) &&
+                    static_cast<uint32_t>(x[1] >> 32) == split_tag(call, slot, 1) &&
+                    static_cast<uint32_t>(x[2] >> 32) == split_tag(call, slot, 2);
+            if (ready) {
+                m = __uint_as_float(static_cast<uint32_t>(x[0]));
+                s = __uint_as_float(static_cast<uint32_t>(x[1]));
+                t = __uint_as_float(static_cast<uint32_t>(x[2]));
+            }
+        }
+        if (__ballot(!ready) == 0) break;
+        if (poll >= max_polls) return true;
+        __builtin_amdgcn_s_sleep(1);
+    }
+    merge_rows16<true>(m, s, t);
+    return false;
+}
+
+struct Split {
+    int n_rows, parts;
+    unsigned long long call;
+    int max_polls;
+};
+
+// Bound by the read of the logits.  NT threads per workgroup (fwd_threads), U
+// 16-byte loads in flight per thread per tile.  A lane's first tile sets its
+// running max; later tiles are accumulated against it (accumulate_at) and take
+// the tile max only when an element lies more than 44 above it.  The chunks left
+// after the full tiles form one predicated tile.
 // The elements outside the row's 16-byte chunks (row_span) are loaded before
 // the first tile and added after the last, one per thread: 4096 rows of 50257
 // logits take 65.6 us (6.28 TB/s) against 81.3 with 2-byte loads throughout.
-template <int NT, int U>
+//
+// One workgroup takes a row, or with kSplit a part of one, where there are too
+// few rows to fill the chip (fwd_parts): part p of row r is workgroup
+// p * n_rows + r.  All but the last part publish their triple and end; the last
+// one, dispatched after them, polls for theirs, merges and writes the row's
+// outputs.  If its polls run out it streams the whole row.
+template <int NT, int U, bool kSplit>
 __global__ __launch_bounds__(NT) void k_lpe_fwd_vec(const uint16_t* __restrict__ logits, int64_t T,
                                                     int64_t V, int64_t stride_b, int64_t stride_t,
                                                     const int64_t* __restrict__ ids, int n_ids,
                                                     float* __restrict__ logp, float* __restrict__ ent,
-                                                    float* __restrict__ lse_out) {
-    const int64_t r = blockIdx.x;
+                                                    float* __restrict__ lse_out, Split sx) {
+    const int part = kSplit ? static_cast<int>(blockIdx.x) / sx.n_rows : 0;
+    const int64_t r = kSplit ? static_cast<int>(blockIdx.x) % sx.n_rows : static_cast<int64_t>(blockIdx.x);
+    const bool last = !kSplit || part + 1 == sx.parts;
     const uint16_t* row = row_ptr(logits, r, T, stride_b, stride_t);
     const RowSpan sp = row_span(row, V);
     const int tid = threadIdx.x;
@@ -114,29 +189,68 @@ __global__ __launch_bounds__(NT) void k_lpe_fwd_vec(const uint16_t* __restrict__
     load_id(row, ids, r, n_ids, V, y, zy);
     bool edge;
     const int64_t e = edge_element(sp, V, tid, edge);
+    edge = edge && last;
     const float z_edge = edge ? bf16_to_f32(row[e]) : 0.f;
 
-    float m = kInit, s = 0.f, t = 0.f;
-    constexpr int64_t kTile = static_cast<int64_t>(NT) * U;
-    const int64_t n_full = sp.n8 / kTile;
-    const v4u* p = sp.body + tid;
-    for (int64_t it = 0; it < n_full; ++it, p += kTile) {
-        v4u v[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) v[u] = __builtin_nontemporal_load(p + u * NT);
-        if (it == 0) {
-            float z[U * 8];
-            unpack(v, z);
-            accumulate(z, m, s, t);
-        } else if (!accumulate_at<true>(v, m, s, t)) {
-            accumulate_exact(v, m, s, t);
-        }
+    const v4u* body = sp.body;
+    int64_t n8 = sp.n8;
+    if constexpr (kSplit) {
+        // Parts of whole 128-byte lines; the last ones may be short or empty.
+        const int64_t per = ((sp.n8 + sx.parts - 1) / sx.parts + 7) / 8 * 8;
+        const int64_t lo = min(part * per, sp.n8);
+        body += lo;
+        n8 = min(per, sp.n8 - lo);
     }
-    const int64_t rem = sp.n8 - n_full * kTile;
-    if (rem > 0) lpe_tail<NT, 1, U>(sp.body + n_full * kTile, rem, tid, m, s, t);
-    accumulate_one(z_edge, edge, m, s, t);
+    float m, s, t;
+    for (;;) {
+        m = kInit, s = 0.f, t = 0.f;
+        constexpr int64_t kTile = static_cast<int64_t>(NT) * U;
+        const int64_t n_full = n8 / kTile;
+        const v4u* p = body + tid;
+        for (int64_t it = 0; it < n_full; ++it, p += kTile) {
+            v4u v[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) v[u] = __builtin_nontemporal_load(p + u * NT);
+            if (it == 0) {
+                float z[U * 8];
+                unpack(v, z);
+                accumulate(z, m, s, t);
+            } else if (!accumulate_at<true>(v, m, s, t)) {
+                accumulate_exact(v, m, s, t);
+            }
+        }
+        const int64_t rem = n8 - n_full * kTile;
+        if (rem > 0) lpe_tail<NT, 1, U>(body + n_full * kTile, rem, tid, m, s, t);
+        accumulate_one(z_edge, edge, m, s, t);
 
-    block_merge<NT>(m, s, t);
+        block_merge<NT>(m, s, t);
+        if constexpr (!kSplit) break;
+        SplitSlot* slots = g_split[sx.call % kSplitRing];
+        if (!last) {
+            if (tid == 0) {
+                const int slot = part * sx.n_rows + static_cast<int>(r);
+                const float v[3] = {m, s, t};
+#pragma unroll
+                for (int w = 0; w < 3; ++w)
+                    __hip_atomic_store(&slots[slot].w[w],
+                                       (static_cast<unsigned long long>(split_tag(sx.call, slot, w)) << 32) |
+                                           __float_as_uint(v[w]),
+                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            return;
+        }
+        if (n8 == sp.n8) break;  // the whole row, after polls that ran out
+        __shared__ int s_gave_up;
+        if (tid < kWave) {
+            const bool gave_up =
+                merge_parts(slots, static_cast<int>(r), sx.n_rows, sx.parts, sx.call, sx.max_polls, m, s, t);
+            if (tid == 0) s_gave_up = gave_up;
+        }
+        __syncthreads();
+        if (!s_gave_up) break;
+        body = sp.body;
+        n8 = sp.n8;
+    }
     finish_row<NT>(r, m, s, t, y, zy, V, n_ids, logp, ent, lse_out);
 }
 
@@ -433,20 +547,56 @@ int fwd_threads(int64_t n, int64_t V) {
     return n <= 256 || (n >= 2048 && V >= 3 * 512 * kFwdUnroll * 8) ? 512 : 256;
 }
 
+// Workgroups per row.  One workgroup to a row is bound by its CU's exponentials
+// (8 of its 11 us for 151936 logits), so rows that leave CUs idle are divided:
+// the kernel alone takes 4.9 us for one row of 151936 logits instead of 10.1,
+// 7.3 for 37 instead of 13.1 and 11.5 for 128 instead of 13.7; 37 rows of 50257
+// 6.0 instead of 7.1.  Two workgroups to a CU are slower (37 rows: 7.9 us, 128:
+// 12.1), as are parts of fewer than 8192 logits, and at 32000 logits the meeting
+// costs what the split gains (37 rows: 5.9 us in 3 parts, 5.5 whole).
+constexpr int64_t kSplitRows = 128;
+constexpr int64_t kSplitWorkgroups = 256;
+constexpr int64_t kSplitMinV = 49152;
+constexpr int64_t kSplitPartV = 8192;
+static_assert(kSplitWorkgroups <= kSplitSlots, "a slot per workgroup");
+
+int fwd_parts(int64_t n, int64_t V) {
+    if (n > kSplitRows || V < kSplitMinV) return 1;
+    return static_cast<int>(std::min<int64_t>({kMaxParts, kSplitWorkgroups / n, V / kSplitPartV}));
+}
+
+// A captured launch would carry one call number into every replay, where the
+// slots of the replay before would pass for its own: it is not split.
+bool capturing(hipStream_t stream) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &status) == hipSuccess) return status != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
+}
+
 int launch_fwd(const uint16_t* logits, int64_t rows, int64_t T, int64_t V, int64_t stride_b,
                int64_t stride_t, const int64_t* ids, int n_ids, float* out, float* entropy, float* lse,
-               hipStream_t stream, const char* who) {
+               hipStream_t stream, const char* who, int max_polls = kSplitPolls) {
     const int64_t n = rows * T;
     if (n == 0) return MESHY_OK;
+    const int parts = fwd_parts(n, V);
+    if (parts > 1 && !capturing(stream)) {
+        static std::atomic<unsigned long long> calls{0};  // the slots' tags tell calls apart
+        const unsigned long long call = calls.fetch_add(1, std::memory_order_relaxed) + 1;
+        hipLaunchKernelGGL((k_lpe_fwd_vec<512, kFwdUnroll, true>), dim3(static_cast<unsigned>(n * parts)), dim3(512), 0,
+                           stream, logits, T, V, stride_b, stride_t, ids, n_ids, out, entropy, lse,
+                           Split{static_cast<int>(n), parts, call, max_polls});
+        return check_launch(who);
+    }
     const dim3 grid(static_cast<unsigned>(n));
     auto go = [&](auto kernel, int threads) {
         hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, stream, logits, T, V, stride_b, stride_t, ids, n_ids, out,
-                           entropy, lse);
+                           entropy, lse, Split{});
     };
     if (fwd_threads(n, V) == 512)
-        go(k_lpe_fwd_vec<512, kFwdUnroll>, 512);
+        go(k_lpe_fwd_vec<512, kFwdUnroll, false>, 512);
     else
-        go(k_lpe_fwd_vec<256, kFwdUnroll>, 256);
+        go(k_lpe_fwd_vec<256, kFwdUnroll, false>, 256);
     return check_launch(who);
 }
 
@@ -529,6 +679,22 @@ extern "C" int meshy_logprob_entropy_fwd(const uint16_t* logits, int64_t rows, i
     if (logp && !labels) return set_error(MESHY_ENULL, "%s: logp needs labels", who);
     return launch_fwd(logits, rows, T, V, stride_b, stride_t, logp ? labels : nullptr, logp ? 1 : 0, logp,
                       entropy, lse, stream, who);
+}
+
+extern "C" int meshy_logprob_entropy_fwd_polls(const uint16_t* logits, int64_t rows, int64_t T, int64_t V,
+                                               int64_t stride_b, int64_t stride_t, const int64_t* labels,
+                                               float* logp, float* entropy, float* lse, int32_t max_polls,
+                                               hipStream_t stream) {
+    using namespace meshy;
+    clear_error();
+    const char* who = "meshy_logprob_entropy_fwd_polls";
+    int rc = check_common(logits, rows, T, V, stride_b, stride_t, who);
+    if (rc) return rc;
+    if (max_polls < 0) return set_error(MESHY_EINVAL, "%s: negative max_polls", who);
+    if (rows * T == 0) return MESHY_OK;
+    if (logp && !labels) return set_error(MESHY_ENULL, "%s: logp needs labels", who);
+    return launch_fwd(logits, rows, T, V, stride_b, stride_t, logp ? labels : nullptr, logp ? 1 : 0, logp,
+                      entropy, lse, stream, who, std::min(max_polls, kSplitPolls));
 }
 
 extern "C" int meshy_gather_logprobs_fwd(const uint16_t* logits, int64_t rows, int64_t T, int64_t V,
