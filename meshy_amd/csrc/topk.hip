@@ -336,6 +336,16 @@ __device__ __forceinline__ bool topk_tile(v4u (&v)[G], OkF ok, int32_t col, bool
     return true;
 }
 
+// m + ln s in double, from the logarithm of s's mantissa (below 1 in magnitude).
+// In fp32 the log-sum-exp of a row of 150 thousand logits lies 3e-7 off by its
+// own rounding, and log2 of an s of 100 adds half of that: the log-probs of the
+// 8 best of 4096 rows of 151936 were 6.9e-8 off 64 bits, and are 2.7e-8 with it.
+__device__ __forceinline__ double lse_of(float m, float s) {
+    int e;
+    const float f = frexpf(s, &e);
+    return static_cast<double>(m) + (static_cast<double>(e) + static_cast<double>(__log2f(f))) * 0.6931471805599453;
+}
+
 // Bound by the read of the logits; NT threads per row as in the log-prob
 // forward.
 template <int NT, int U, int CAP>
@@ -350,7 +360,7 @@ __global__ __launch_bounds__(NT) void k_topk_vec(const uint16_t* __restrict__ lo
     __shared__ uint16_t s_key[kKeyRows][kWave];  // the waves' chunks, then the row's head and tail elements
     __shared__ uint64_t s_list[kMaxListed];
     __shared__ int s_listed;
-    __shared__ float s_lse;
+    __shared__ double s_lse;
     const int64_t r = blockIdx.x;
     const uint16_t* row = row_ptr(logits, r, T, stride_b, stride_t);
     const RowSpan sp = row_span(row, V);
@@ -467,12 +477,10 @@ __global__ __launch_bounds__(NT) void k_topk_vec(const uint16_t* __restrict__ lo
         // torch.logsumexp: NaN for a row holding NaN; otherwise +inf for a row
         // whose max is +inf (its candidates' log-probs are then NaN for the
         // +inf logit and -inf for finite ones), where s is NaN.
-        const float lse = __ballot(nan) ? __builtin_nanf("")
-                          : m == __builtin_inff() ? m
-                                                  : fmaf(__log2f(s), kLn2, m);
+        const double lse = __ballot(nan) ? __builtin_nan("") : m == __builtin_inff() ? __builtin_inf() : lse_of(m, s);
         if (tid == 0) {
             s_lse = lse;
-            if (lse_out) lse_out[r] = lse;
+            if (lse_out) lse_out[r] = static_cast<float>(lse);
         }
     }
     __syncthreads();
@@ -520,7 +528,7 @@ __global__ __launch_bounds__(NT) void k_topk_vec(const uint16_t* __restrict__ lo
         __syncthreads();
     }
     const int listed = s_listed;
-    const float lse = s_lse;
+    const double lse = s_lse;
     for (int i = tid; i < listed; i += NT) {
         const uint64_t own = s_list[i];
         int rank = 0;
@@ -528,7 +536,7 @@ __global__ __launch_bounds__(NT) void k_topk_vec(const uint16_t* __restrict__ lo
         for (int j = 0; j < listed; ++j) rank += s_list[j] > own;
         if (rank < k) {
             ids[r * k + rank] = static_cast<int32_t>(~static_cast<uint32_t>(own));
-            lps[r * k + rank] = value_of(static_cast<uint32_t>(own >> 32)) - lse;
+            lps[r * k + rank] = static_cast<float>(value_of(static_cast<uint32_t>(own >> 32)) - lse);
         }
     }
 }
