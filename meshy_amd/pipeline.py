@@ -59,13 +59,16 @@ class RaggedSamples:
         lay.add("rewards", max(n, 1), torch.float32)
         lay.add("group_off", n_groups + 1, torch.int64)
         lay.add("pos_w", max(n, 1), torch.float32)
+        # Everything above is the samples' and goes to the device as soon as a
+        # pack starts; the plan tables below follow once they are computed.
+        self.tables_at = lay.size
         # plan tables of one rank: at most n micros and n documents
         lay.add("seq", max(n, 1), torch.int64)
         lay.add("out_off", n + 1, torch.int64)
         lay.add("doc_len", max(n, 1), torch.int64)
         lay.add("doc_start", n + 1, torch.int32)
         lay.add("doc_sample", max(n, 1), torch.int32)
-        self.adv_at = lay.size  # the copy ends here
+        self.adv_at = lay.size  # the second copy ends here
         lay.add("adv_samples", max(n, 1), torch.float32)  # written on the device, last
         self.lay = lay
         self.n_groups = n_groups
@@ -73,7 +76,7 @@ class RaggedSamples:
         self.buf = torch.empty(lay.size, dtype=torch.uint8, pin_memory=torch.cuda.is_available())
         self._np_buf = self.buf.numpy()
         self._np: dict[str, np.ndarray] = {}
-        self.copied = None  # event of the last copy out of buf
+        self.copied = None  # event of the last copy of the plan tables out of buf
         self._step_args = None  # meshy_step_plan's struct over this buffer
         self._cfg_key = None  # the settings last written into it
         self._stream = None  # (raw handle, torch Stream) of the last copy's stream
@@ -259,12 +262,11 @@ def pack_step(ragged: RaggedSamples, cfg: PlannerConfig, device, *, dp_size: int
               with_plan_objects: bool = False, broadcast_advantages: bool = True) -> PackResult:
     """Plan, copy, normalise rewards and build every micro of ``rank``.
 
-    One native call (``meshy_step_plan``) counts the loss tokens, plans and
-    writes this rank's pack tables into the staging buffer behind the samples;
-    one copy takes both to the device.  (Copying the samples before the plan,
-    so that the copy runs beside it, costs a second copy and takes longer at
-    every size: 45.7 against 41.9 us for 16 samples, 57.4 against 54.8 for 64,
-    94.7 against 93.1 for 256, and for 1024 313 against 304 waited for.)
+    The samples' part of the staging buffer is copied to the device first and
+    the GRPO kernel queued behind it, so both run while the host plans.  One
+    native call
+    (``meshy_step_plan``) counts the loss tokens, plans and writes this rank's
+    pack tables into the staging buffer; they follow in a second, small copy.
     The Plan dataclasses are built when ``PackResult.plan`` is first read
     (``with_plan_objects`` builds them here)."""
     device = torch.device(device)
@@ -274,11 +276,22 @@ def pack_step(ragged: RaggedSamples, cfg: PlannerConfig, device, *, dp_size: int
     dbuf = torch.empty(lay.size, dtype=torch.uint8, device=device)
     base = dbuf.data_ptr()
     hbase = ragged.buf.data_ptr()
+    cut = ragged.tables_at
+    # Raw asynchronous copies from the pinned buffer, on the device's current
+    # stream; the buffer outlives them (ragged.copied marks the second).
     if dp_size <= 0 or ragged.n % dp_size != 0:
         raise ValueError(
             f"batch size {ragged.n} is not divisible by DP size {dp_size}; adjust "
             "rollout.batch_size * group_size to a multiple of dp_replicate * dp_shard"
         )
+    _lib.check(lib.meshy_copy_to_device(base, hbase, cut, handle), "meshy_copy_to_device")
+    # GRPO reads only the rewards and group offsets of the first copy: it runs
+    # while the host plans.  Its output region lies past the plan tables, so
+    # the second copy stops short of it.
+    adv = lay.addr(base, "adv_samples")
+    rc = lib.meshy_grpo_advantage(lay.addr(base, "rewards"), ragged.n, lay.addr(base, "group_off"), ragged.n_groups,
+                                  adv, handle)
+    _lib.check(rc, "meshy_grpo_advantage")
     if ragged.copied is not None:
         ragged.copied.synchronize()  # the tables below reuse the pinned buffer the last copy read
     t = PlanTables(ragged.n, dp_size, cfg.mini_batch_size)
@@ -287,15 +300,8 @@ def pack_step(ragged: RaggedSamples, cfg: PlannerConfig, device, *, dp_size: int
     t.n_micro_total = int(a.plan.n_micro_total)
     nm, nd_total = int(a.n_micro), int(a.n_docs)
 
-    # A raw asynchronous copy from the pinned buffer, on the device's current
-    # stream; the buffer outlives it (ragged.copied marks its end).  GRPO's output
-    # region lies past the copied ones.
-    _lib.check(lib.meshy_copy_to_device(base, hbase, ragged.adv_at, handle), "meshy_copy_to_device")
+    _lib.check(lib.meshy_copy_to_device(base + cut, hbase + cut, ragged.adv_at - cut, handle), "meshy_copy_to_device")
     ragged.record_copy(device)
-    adv = lay.addr(base, "adv_samples")
-    rc = lib.meshy_grpo_advantage(lay.addr(base, "rewards"), ragged.n, lay.addr(base, "group_off"), ragged.n_groups,
-                                  adv, handle)
-    _lib.check(rc, "meshy_grpo_advantage")
 
     seq = ragged.np_view("seq")[:nm]
     start = ragged.np_view("doc_start")[:nm + 1]
