@@ -534,10 +534,11 @@ int check_common(const void* logits, int64_t rows, int64_t T, int64_t V, int64_t
     return MESHY_OK;
 }
 
-// Threads of a row's workgroup.  Up to 256 rows there is one workgroup per CU
-// at most, and a CU streams in proportion to its loads in flight: 512 threads
-// take 13.0 us for 37 rows of 151936 logits and 16.0 for 256, against 19.1 and
-// 21.1 with 256 threads (1024 threads: 12.4 and 16.3).  From 257 rows on, 256
+// Threads of a workgroup that takes a whole row.  Up to 256 rows there is one
+// workgroup per CU at most, and a CU streams in proportion to its loads in
+// flight: 512 threads take 13.0 us for 37 undivided rows of 151936 logits and
+// 16.0 for 256, against 19.1 and 21.1 with 256 threads (1024 threads: 12.4 and
+// 16.3).  From 257 rows on, 256
 // threads spread the rows more evenly (512 rows: 27.4 against 28.1 us; 4096
 // rows of 50257: 65.6 against 72.2, where most of a row is the predicated last
 // tile of 4096 chunks).  Many rows of at least 3 full tiles of 512 threads
