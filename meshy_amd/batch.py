@@ -232,7 +232,10 @@ def _gather_column(samples: Sequence[Any], used: np.ndarray, used_b: bytes, need
 
 @dataclass
 class PackJob:
-    """Device-resident inputs of one pack launch (see ``stage_micro_batches``)."""
+    """Device-resident inputs of one pack launch (see ``stage_micro_batches``).
+
+    The micros' views are made from the arrays below when a batch first needs
+    them: the job owns them, none lies in memory that a later call rewrites."""
 
     micros: tuple
     layout: str
@@ -259,6 +262,8 @@ class PackJob:
     teacher_k: int = 0
     #: The staged mask holds one byte per token (0 or 1) instead of fp32.
     mask_u8: bool = False
+    #: Pinned staging buffer kept alive while its copies may still be queued.
+    host: torch.Tensor | None = None
     #: Per micro, whether its advantages are per token (None: every micro
     #: with documents, when per_token_adv).
     per_token_micros: tuple | None = None
@@ -779,6 +784,7 @@ class _PackViews:
         self.version0 = obuf._version
         self.pos_w_src = (lay, dbuf)
         self._job = job
+        self.n_out = int(job.out_off[-1])  # elements of each per-token output
         self.doc_start = job.doc_start.tolist()
         self.nd = [b - a for a, b in zip(self.doc_start, self.doc_start[1:])]
         self.micros = job.micros
@@ -846,7 +852,7 @@ class _PackViews:
             specs = tuple((regions[name][0], _SCALAR_TYPE[regions[name][2]]) if name in regions else None
                           for name in self._TOK)
             rows, seq = (np.asarray(x, np.int64).tobytes() for x in (self._job.rows, self._job.seq))
-            self._tok = _lib.stage().token_views(self.obuf, specs, rows, seq)
+            self._tok = _lib.stage().token_views(self.obuf, specs, rows, seq, self.n_out)
         return self._tok
 
     def tokens(self, mb: "PackedBatch", f: dict) -> None:

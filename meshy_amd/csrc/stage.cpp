@@ -53,13 +53,15 @@
 //       for an absent region), the four tables as bytes, and the compact
 //       sample map with each used sample's prefix length as plan_tables
 //       gives them.
-//   token_views(buf, regions, rows, seq)
+//   token_views(buf, regions, rows, seq[, elements])
 //       The per-token tensors of every micro of a pack launch: regions is one
 //       (byte offset in buf, c10::ScalarType) or None per output, rows and seq
 //       the micros' shapes as int64 bytes; returns one tuple per micro of its
 //       [rows, seq] tensors (None for an absent output).  A micro's elements
-//       follow the previous micro's in each region.  The tensors share buf's
-//       storage and version counter, as buf[a:b].view(dtype) would.
+//       follow the previous micro's in each region; with `elements`, every
+//       region's length, the micros must fill it exactly (as torch.split
+//       requires).  The tensors share buf's storage and version counter, as
+//       buf[a:b].view(dtype) would.
 #include <Python.h>
 
 #include <torch/csrc/Exceptions.h>
@@ -693,8 +695,9 @@ at::Tensor typed_view(const at::Tensor& buf, caffe2::TypeMeta type, int64_t offs
 PyObject* token_views(PyObject*, PyObject* args) {
     HANDLE_TH_ERRORS
     PyObject *py_buf, *py_regions, *py_rows, *py_seq;
-    if (!PyArg_ParseTuple(args, "OO!O!O!", &py_buf, &PyTuple_Type, &py_regions, &PyBytes_Type, &py_rows,
-                          &PyBytes_Type, &py_seq))
+    long long elements = -1;
+    if (!PyArg_ParseTuple(args, "OO!O!O!|L", &py_buf, &PyTuple_Type, &py_regions, &PyBytes_Type, &py_rows,
+                          &PyBytes_Type, &py_seq, &elements))
         return nullptr;
     if (!THPVariable_Check(py_buf)) {
         PyErr_SetString(PyExc_TypeError, "token_views: buf must be a tensor");
@@ -712,6 +715,8 @@ PyObject* token_views(PyObject*, PyObject* args) {
         TORCH_CHECK_VALUE(rows[k] >= 0 && seq[k] >= 0, "token_views: negative sizes");
         total += rows[k] * seq[k];
     }
+    TORCH_CHECK_VALUE(elements < 0 || total == elements, "token_views: the micros hold ", total,
+                      " elements, each output has ", elements);
     const Py_ssize_t n_out = PyTuple_GET_SIZE(py_regions);
     struct Region {
         caffe2::TypeMeta type;

@@ -303,17 +303,19 @@ def pack_step(ragged: RaggedSamples, cfg: PlannerConfig, device, *, dp_size: int
     _lib.check(lib.meshy_copy_to_device(base + cut, hbase + cut, ragged.adv_at - cut, handle), "meshy_copy_to_device")
     ragged.record_copy(device)
 
-    seq = ragged.np_view("seq")[:nm]
-    start = ragged.np_view("doc_start")[:nm + 1]
-    out_off = ragged.np_view("out_off")[:nm + 1]
+    # Copies: the next step rewrites the pinned tables, and a batch reads these
+    # when one of its fields is first read.
+    seq = ragged.np_view("seq")[:nm].copy()
+    start = ragged.np_view("doc_start")[:nm + 1].copy()
+    out_off = ragged.np_view("out_off")[:nm + 1].copy()
     packed = cfg.layout == "packed"
     job = PackJob.fast(
-        micros=_LiteMicros(seq, start, ragged.np_view("doc_len")[:nd_total]),
+        micros=_LiteMicros(seq, start, ragged.np_view("doc_len")[:nd_total].copy()),
         layout=cfg.layout, device=device, dbuf=dbuf, lay=lay,
         need_rollout_lp=ragged.need_rollout_lp, per_token_adv=False, n_samples=ragged.n, seq=seq,
         rows=np.ones(nm, np.int64) if packed else np.maximum(np.diff(start), 1), out_off=out_off, doc_start=start,
         max_elems=int(a.max_micro_elems), max_docs=int(a.max_docs_per_micro), adv_samples=adv,
-        broadcast_advantages=broadcast_advantages, stream=handle, mask_u8=ragged.mask_u8,
+        broadcast_advantages=broadcast_advantages, stream=handle, mask_u8=ragged.mask_u8, host=ragged.buf,
     )
     batches = launch_pack(job)
     return PackResult(tables_to_plan(t) if with_plan_objects else None, t, batches, (dbuf, lay, ragged.n))
@@ -321,8 +323,8 @@ def pack_step(ragged: RaggedSamples, cfg: PlannerConfig, device, *, dp_size: int
 
 class _LiteMicros:
     """The micros of a step as ``launch_pack`` reads them, each made on first
-    use from the plan's tables (numpy views, read as lists the first time a
-    micro is needed; no dataclass per micro)."""
+    use from the plan's tables (arrays that nothing rewrites, read as lists the
+    first time a micro is needed; no dataclass per micro)."""
 
     __slots__ = ("_arrays", "_lists", "_n", "_made")
 
