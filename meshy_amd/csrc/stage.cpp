@@ -64,6 +64,7 @@
 //       buf[a:b].view(dtype) would.
 #include <Python.h>
 
+#include <c10/core/InferenceMode.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -742,6 +743,9 @@ PyObject* token_views(PyObject*, PyObject* args) {
     }
     PyObject* out = PyList_New(n_micro);
     if (!out) return nullptr;
+    // The views are of the buffer's kind, as a slice's would be, not of the
+    // caller's mode: a batch first read while scoring is trained on later.
+    c10::InferenceMode mode(buf.is_inference());
     int64_t at = 0;
     for (Py_ssize_t k = 0; k < n_micro; ++k) {
         PyObject* t = PyTuple_New(n_out);

@@ -66,3 +66,20 @@ def test_bad_arguments_are_refused():
         _views(np.zeros(64, np.uint8), ((0, 4),), [1], [1])
     with pytest.raises(ValueError):
         _views(torch.zeros(64), ((0, 4),), [1], [1])
+
+
+@pytest.mark.parametrize("made_in", [False, True])
+@pytest.mark.parametrize("read_in", [False, True])
+def test_views_are_of_the_buffers_kind_whatever_the_mode(made_in, read_in):
+    with torch.inference_mode(made_in):
+        buf = torch.zeros(512, dtype=torch.uint8)
+    with torch.inference_mode(read_in):
+        (t, u), = _views(buf, ((0, _SCALAR_TYPE[torch.float32]), (256, _SCALAR_TYPE[torch.int64])), [1], [32])
+    assert t.is_inference() == u.is_inference() == made_in
+    if not made_in:  # read while scoring, trained on later
+        before = buf._version
+        t.add_(1)
+        assert buf._version == u._version == before + 1
+        w = torch.ones(1, 32, requires_grad=True)
+        (w * t).sum().backward()
+        assert torch.equal(w.grad, torch.ones(1, 32))
