@@ -571,6 +571,9 @@ typedef struct meshy_gae_args {
     const int64_t* seg_offsets;    /* nullable, see above                     */
 } meshy_gae_args;
 
+/* Under stream capture the call also records a small kernel that clears its
+ * slots in the workspace, so that a replay takes none of the replay before; the
+ * graph reads every argument array, seg_offsets and lengths too, on each replay. */
 size_t meshy_gae_workspace_size(int64_t rows, int64_t S, int64_t n_docs);
 int meshy_gae(const meshy_gae_args* args, hipStream_t stream);
 

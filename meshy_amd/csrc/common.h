@@ -12,6 +12,17 @@ namespace meshy {
 // Checks the launch that was just enqueued; maps a HIP error to its positive code.
 int check_launch(const char* what);
 
+// Whether the stream is being captured (or cannot be asked).  Kernels that meet
+// in memory under a number drawn per call need another route there: a captured
+// launch carries one number into every replay, where what the replay before
+// left would pass for its own.
+inline bool capturing(hipStream_t stream) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &status) == hipSuccess) return status != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
+}
+
 constexpr int kWave = 64;
 
 __device__ __forceinline__ float bf16_lo(uint32_t w) { return __uint_as_float(w << 16); }

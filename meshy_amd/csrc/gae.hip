@@ -976,6 +976,15 @@ int gae_launch(const meshy_gae_args& g, hipStream_t stream) {
                      (!g.adv || al16(g.adv)) && (!g.returns || al16(g.returns));
     if (nc > 0 && (g.adv || g.returns)) {
         const unsigned long long epoch = g_gae_epoch.fetch_add(1, std::memory_order_relaxed) + 1;
+        // Every replay of a captured call carries the same epoch: the slots are
+        // cleared in the graph (a clear word's tag, 0, is no call's but by a
+        // 2^-128 coincidence of a slot's four words).
+        if (capturing(stream)) {
+            const int64_t words = nc * static_cast<int64_t>(sizeof(Slot) / sizeof(float));
+            hipLaunchKernelGGL(k_gae_zero, dim3(static_cast<unsigned>(ceil_div(words, kThreads))), dim3(kThreads), 0,
+                               stream, reinterpret_cast<float*>(ws.slot), words);
+            if ((rc = check_launch("meshy_gae(slots)"))) return rc;
+        }
         hipLaunchKernelGGL(k_gae_scan, dim3(static_cast<unsigned>(nc)), dim3(kThreads), 0, stream, g, ws, n, nc, vec,
                            epoch, g_gae_max_polls.load(std::memory_order_relaxed));
         if ((rc = check_launch("meshy_gae(scan)"))) return rc;

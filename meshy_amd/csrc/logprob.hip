@@ -566,22 +566,13 @@ int fwd_parts(int64_t n, int64_t V) {
     return static_cast<int>(std::min<int64_t>({kMaxParts, kSplitWorkgroups / n, V / kSplitPartV}));
 }
 
-// A captured launch would carry one call number into every replay, where the
-// slots of the replay before would pass for its own: it is not split.
-bool capturing(hipStream_t stream) {
-    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &status) == hipSuccess) return status != hipStreamCaptureStatusNone;
-    (void)hipGetLastError();
-    return true;
-}
-
 int launch_fwd(const uint16_t* logits, int64_t rows, int64_t T, int64_t V, int64_t stride_b,
                int64_t stride_t, const int64_t* ids, int n_ids, float* out, float* entropy, float* lse,
                hipStream_t stream, const char* who, int max_polls = kSplitPolls) {
     const int64_t n = rows * T;
     if (n == 0) return MESHY_OK;
     const int parts = fwd_parts(n, V);
-    if (parts > 1 && !capturing(stream)) {
+    if (parts > 1 && !capturing(stream)) {  // else a replay would take the slots of the one before
         static std::atomic<unsigned long long> calls{0};  // the slots' tags tell calls apart
         const unsigned long long call = calls.fetch_add(1, std::memory_order_relaxed) + 1;
         hipLaunchKernelGGL((k_lpe_fwd_vec<512, kFwdUnroll, true>), dim3(static_cast<unsigned>(n * parts)), dim3(512), 0,
