@@ -304,8 +304,10 @@ int meshy_logprob_entropy_fwd(const uint16_t* logits, int64_t rows, int64_t T, i
                               float* logp, float* entropy, float* lse, hipStream_t stream);
 /* Test hook, no counterpart in the reference: the same call, in which a
  * workgroup that waits for the other parts of its row (few rows are divided
- * over several workgroups) polls max_polls times (0 to the default of 4000)
- * before it streams the whole row itself. */
+ * over several workgroups) looks max_polls times (0, not once, to the default
+ * of 4000) before it streams those parts itself.  The results have the same
+ * bits either way; on a stream that is being captured rows are not divided,
+ * and their last bits may differ from an uncaptured call's. */
 int meshy_logprob_entropy_fwd_polls(const uint16_t* logits, int64_t rows, int64_t T, int64_t V,
                                     int64_t stride_b, int64_t stride_t, const int64_t* labels,
                                     float* logp, float* entropy, float* lse, int32_t max_polls,
@@ -362,6 +364,10 @@ int meshy_logprob_bwd_noalloc(const uint16_t* logits, int64_t rows, int64_t T, i
 int meshy_gather_logprobs_fwd(const uint16_t* logits, int64_t rows, int64_t T, int64_t V,
                               int64_t stride_b, int64_t stride_t, const int64_t* ids,
                               int64_t n_ids, float* out, float* lse, hipStream_t stream);
+/* Test hook, as meshy_logprob_entropy_fwd_polls. */
+int meshy_gather_logprobs_fwd_polls(const uint16_t* logits, int64_t rows, int64_t T, int64_t V,
+                                    int64_t stride_b, int64_t stride_t, const int64_t* ids, int64_t n_ids,
+                                    float* out, float* lse, int32_t max_polls, hipStream_t stream);
 int meshy_gather_logprobs_bwd(const uint16_t* logits, int64_t rows, int64_t T, int64_t V,
                               int64_t stride_b, int64_t stride_t, const int64_t* ids,
                               int64_t n_ids, const float* lse, const float* grad_out,

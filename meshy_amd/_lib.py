@@ -297,6 +297,11 @@ SIGNATURES = {
         [c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64, c_void_p, c_int64, c_void_p,
          c_void_p, c_void_p],
     ),
+    "meshy_gather_logprobs_fwd_polls": (
+        c_int,
+        [c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64, c_void_p, c_int64, c_void_p,
+         c_void_p, c_int32, c_void_p],
+    ),
     "meshy_gather_logprobs_bwd": (
         c_int,
         [c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64, c_void_p, c_int64, c_void_p,

@@ -99,7 +99,7 @@ __device__ __forceinline__ void accumulate_exact(v4u (&v)[U], float& m, float& s
 // when its tag is the call's; whatever else the slot held carries another tag,
 // and nothing is cleared.  Call e uses entry e % kSplitRing: a call overlapped
 // by a later one of the same entry (kSplitRing calls on, on another stream) can
-// lose a word, and then streams the whole row itself.
+// lose a word, and then streams the row's other parts itself.
 constexpr int kMaxParts = 16;     // merged in one row of 16 lanes
 constexpr int kSplitSlots = 256;  // at least a launch's rows * parts
 constexpr int kSplitRing = 64;
@@ -118,18 +118,22 @@ __device__ __forceinline__ uint32_t split_tag(unsigned long long call, int slot,
     return static_cast<uint32_t>(x >> 32);
 }
 
-// A split row's part merged with the others (wave 0 holds this part's triple in
-// lane 0): polls for the triples of parts 0 .. parts - 2 of row r and merges in
-// a fixed order, the result in lane 0.  Returns whether the polls ran out first.
-__device__ __forceinline__ bool merge_parts(const SplitSlot* slots, int r, int n_rows, int parts,
-                                            unsigned long long call, int max_polls, float& m, float& s, float& t) {
+// Merges the triples of a row's parts, part p in lane p, in a fixed order; the
+// result in lane 0.
+__device__ __forceinline__ void merge_parts(int parts, float& m, float& s, float& t) {
+    const bool in = static_cast<int>(threadIdx.x) < parts;
+    m = in ? m : kInit, s = in ? s : 0.f, t = in ? t : 0.f;
+    merge_rows16<true>(m, s, t);
+}
+
+// Wave 0 polls, max_polls times at most, for the triples of parts 0 ..
+// parts - 2 of row r, part p's in lane p.  Returns whether the polls ran out.
+__device__ __forceinline__ bool poll_parts(const SplitSlot* slots, int r, int n_rows, int parts,
+                                           unsigned long long call, int max_polls, float& m, float& s, float& t) {
     const int lane = threadIdx.x;
-    const bool own = lane + 1 == parts;
-    const float m0 = lane_f32(m, 0), s0 = lane_f32(s, 0), t0 = lane_f32(t, 0);
-    m = own ? m0 : kInit, s = own ? s0 : 0.f, t = own ? t0 : 0.f;
     const int slot = lane * n_rows + r;
     bool ready = lane + 1 >= parts;
-    for (int poll = 0;; ++poll) {
+    for (int poll = 0; poll < max_polls; ++poll) {
         if (!ready) {
             unsigned long long x[3];
 #pragma unroll
@@ -144,12 +148,10 @@ __device__ __forceinline__ bool merge_parts(const SplitSlot* slots, int r, int n
                 t = __uint_as_float(static_cast<uint32_t>(x[2]));
             }
         }
-        if (__ballot(!ready) == 0) break;
-        if (poll >= max_polls) return true;
+        if (__ballot(!ready) == 0) return false;
         __builtin_amdgcn_s_sleep(1);
     }
-    merge_rows16<true>(m, s, t);
-    return false;
+    return true;
 }
 
 struct Split {
@@ -171,7 +173,8 @@ struct Split {
 // few rows to fill the chip (fwd_parts): part p of row r is workgroup
 // p * n_rows + r.  All but the last part publish their triple and end; the last
 // one, dispatched after them, polls for theirs, merges and writes the row's
-// outputs.  If its polls run out it streams the whole row.
+// outputs.  If its polls run out it streams the other parts itself, part by
+// part, so that the result has the same bits whoever took them.
 template <int NT, int U, bool kSplit>
 __global__ __launch_bounds__(NT) void k_lpe_fwd_vec(const uint16_t* __restrict__ logits, int64_t T,
                                                     int64_t V, int64_t stride_b, int64_t stride_t,
@@ -192,25 +195,25 @@ __global__ __launch_bounds__(NT) void k_lpe_fwd_vec(const uint16_t* __restrict__
     edge = edge && last;
     const float z_edge = edge ? bf16_to_f32(row[e]) : 0.f;
 
-    const v4u* body = sp.body;
-    int64_t n8 = sp.n8;
-    if constexpr (kSplit) {
-        // Parts of whole 128-byte lines; the last ones may be short or empty.
-        const int64_t per = ((sp.n8 + sx.parts - 1) / sx.parts + 7) / 8 * 8;
-        const int64_t lo = min(part * per, sp.n8);
-        body += lo;
-        n8 = min(per, sp.n8 - lo);
-    }
     float m, s, t;
-    for (;;) {
+    for (int p = part;;) {
+        const v4u* body = sp.body;
+        int64_t n8 = sp.n8;
+        if constexpr (kSplit) {
+            // Parts of whole 128-byte lines; the last ones may be short or empty.
+            const int64_t per = ((sp.n8 + sx.parts - 1) / sx.parts + 7) / 8 * 8;
+            const int64_t lo = min(p * per, sp.n8);
+            body += lo;
+            n8 = min(per, sp.n8 - lo);
+        }
         m = kInit, s = 0.f, t = 0.f;
         constexpr int64_t kTile = static_cast<int64_t>(NT) * U;
         const int64_t n_full = n8 / kTile;
-        const v4u* p = body + tid;
-        for (int64_t it = 0; it < n_full; ++it, p += kTile) {
+        const v4u* c = body + tid;
+        for (int64_t it = 0; it < n_full; ++it, c += kTile) {
             v4u v[U];
 #pragma unroll
-            for (int u = 0; u < U; ++u) v[u] = __builtin_nontemporal_load(p + u * NT);
+            for (int u = 0; u < U; ++u) v[u] = __builtin_nontemporal_load(c + u * NT);
             if (it == 0) {
                 float z[U * 8];
                 unpack(v, z);
@@ -221,35 +224,51 @@ __global__ __launch_bounds__(NT) void k_lpe_fwd_vec(const uint16_t* __restrict__
         }
         const int64_t rem = n8 - n_full * kTile;
         if (rem > 0) lpe_tail<NT, 1, U>(body + n_full * kTile, rem, tid, m, s, t);
-        accumulate_one(z_edge, edge, m, s, t);
+        accumulate_one(z_edge, edge && p == part, m, s, t);
 
         block_merge<NT>(m, s, t);
-        if constexpr (!kSplit) break;
-        SplitSlot* slots = g_split[sx.call % kSplitRing];
-        if (!last) {
-            if (tid == 0) {
-                const int slot = part * sx.n_rows + static_cast<int>(r);
-                const float v[3] = {m, s, t};
+        if constexpr (!kSplit) {
+            break;
+        } else {
+            SplitSlot* slots = g_split[sx.call % kSplitRing];
+            if (!last) {
+                if (tid == 0) {
+                    const int slot = part * sx.n_rows + static_cast<int>(r);
+                    const float v[3] = {m, s, t};
 #pragma unroll
-                for (int w = 0; w < 3; ++w)
-                    __hip_atomic_store(&slots[slot].w[w],
-                                       (static_cast<unsigned long long>(split_tag(sx.call, slot, w)) << 32) |
-                                           __float_as_uint(v[w]),
-                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    for (int w = 0; w < 3; ++w)
+                        __hip_atomic_store(&slots[slot].w[w],
+                                           (static_cast<unsigned long long>(split_tag(sx.call, slot, w)) << 32) |
+                                               __float_as_uint(v[w]),
+                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+                return;
             }
-            return;
+            __shared__ float s_part[kMaxParts][3];
+            __shared__ int s_gave_up;
+            if (tid < kWave) {
+                if (tid == 0) s_part[p][0] = m, s_part[p][1] = s, s_part[p][2] = t;
+                if (p == part) {  // the workgroup's own
+                    const float own[3] = {lane_f32(m, 0), lane_f32(s, 0), lane_f32(t, 0)};
+                    const bool gave_up = poll_parts(slots, static_cast<int>(r), sx.n_rows, sx.parts, sx.call,
+                                                    sx.max_polls, m, s, t);
+                    if (tid == part) m = own[0], s = own[1], t = own[2];
+                    if (tid == 0) s_gave_up = gave_up;
+                }
+            }
+            __syncthreads();  // also keeps block_merge's scratch for the next part
+            if (p == part ? !s_gave_up : p + 2 == sx.parts) {
+                if (tid < kWave) {
+                    if (p != part) {
+                        const float* q = s_part[min(tid, part)];
+                        m = q[0], s = q[1], t = q[2];
+                    }
+                    merge_parts(sx.parts, m, s, t);
+                }
+                break;
+            }
+            p = p == part ? 0 : p + 1;
         }
-        if (n8 == sp.n8) break;  // the whole row, after polls that ran out
-        __shared__ int s_gave_up;
-        if (tid < kWave) {
-            const bool gave_up =
-                merge_parts(slots, static_cast<int>(r), sx.n_rows, sx.parts, sx.call, sx.max_polls, m, s, t);
-            if (tid == 0) s_gave_up = gave_up;
-        }
-        __syncthreads();
-        if (!s_gave_up) break;
-        body = sp.body;
-        n8 = sp.n8;
     }
     finish_row<NT>(r, m, s, t, y, zy, V, n_ids, logp, ent, lse_out);
 }
@@ -568,11 +587,15 @@ int fwd_parts(int64_t n, int64_t V) {
 
 int launch_fwd(const uint16_t* logits, int64_t rows, int64_t T, int64_t V, int64_t stride_b,
                int64_t stride_t, const int64_t* ids, int n_ids, float* out, float* entropy, float* lse,
-               hipStream_t stream, const char* who, int max_polls = kSplitPolls) {
+               hipStream_t stream, const char* who, int max_polls) {
     const int64_t n = rows * T;
     if (n == 0) return MESHY_OK;
     const int parts = fwd_parts(n, V);
-    if (parts > 1 && !capturing(stream)) {  // else a replay would take the slots of the one before
+    // A replay would take the slots of the one before: a captured call is not
+    // divided (its last bits may then differ; the last part's workgroups taking
+    // every part in turn gives the same ones in 19 us for 37 rows of 151936
+    // logits and 32 for one, where whole rows take 10.6 and 10.2).
+    if (parts > 1 && !capturing(stream)) {
         static std::atomic<unsigned long long> calls{0};  // the slots' tags tell calls apart
         const unsigned long long call = calls.fetch_add(1, std::memory_order_relaxed) + 1;
         hipLaunchKernelGGL((k_lpe_fwd_vec<512, kFwdUnroll, true>), dim3(static_cast<unsigned>(n * parts)), dim3(512), 0,
@@ -658,28 +681,13 @@ int launch_bwd(const uint16_t* logits, int64_t rows, int64_t T, int64_t V, int64
 }  // namespace
 }  // namespace meshy
 
-extern "C" int meshy_logprob_entropy_fwd(const uint16_t* logits, int64_t rows, int64_t T, int64_t V,
-                                         int64_t stride_b, int64_t stride_t, const int64_t* labels,
-                                         float* logp, float* entropy, float* lse,
-                                         hipStream_t stream) {
-    using namespace meshy;
-    clear_error();
-    const char* who = "meshy_logprob_entropy_fwd";
-    int rc = check_common(logits, rows, T, V, stride_b, stride_t, who);
-    if (rc) return rc;
-    if (rows * T == 0) return MESHY_OK;
-    if (logp && !labels) return set_error(MESHY_ENULL, "%s: logp needs labels", who);
-    return launch_fwd(logits, rows, T, V, stride_b, stride_t, logp ? labels : nullptr, logp ? 1 : 0, logp,
-                      entropy, lse, stream, who);
-}
+namespace meshy {
+namespace {
 
-extern "C" int meshy_logprob_entropy_fwd_polls(const uint16_t* logits, int64_t rows, int64_t T, int64_t V,
-                                               int64_t stride_b, int64_t stride_t, const int64_t* labels,
-                                               float* logp, float* entropy, float* lse, int32_t max_polls,
-                                               hipStream_t stream) {
-    using namespace meshy;
+int entropy_fwd(const uint16_t* logits, int64_t rows, int64_t T, int64_t V, int64_t stride_b, int64_t stride_t,
+                const int64_t* labels, float* logp, float* entropy, float* lse, int32_t max_polls,
+                hipStream_t stream, const char* who) {
     clear_error();
-    const char* who = "meshy_logprob_entropy_fwd_polls";
     int rc = check_common(logits, rows, T, V, stride_b, stride_t, who);
     if (rc) return rc;
     if (max_polls < 0) return set_error(MESHY_EINVAL, "%s: negative max_polls", who);
@@ -689,21 +697,54 @@ extern "C" int meshy_logprob_entropy_fwd_polls(const uint16_t* logits, int64_t r
                       entropy, lse, stream, who, std::min(max_polls, kSplitPolls));
 }
 
-extern "C" int meshy_gather_logprobs_fwd(const uint16_t* logits, int64_t rows, int64_t T, int64_t V,
-                                         int64_t stride_b, int64_t stride_t, const int64_t* ids,
-                                         int64_t n_ids, float* out, float* lse, hipStream_t stream) {
-    using namespace meshy;
+int gather_fwd(const uint16_t* logits, int64_t rows, int64_t T, int64_t V, int64_t stride_b, int64_t stride_t,
+               const int64_t* ids, int64_t n_ids, float* out, float* lse, int32_t max_polls, hipStream_t stream,
+               const char* who) {
     clear_error();
-    const char* who = "meshy_gather_logprobs_fwd";
     int rc = check_common(logits, rows, T, V, stride_b, stride_t, who);
     if (rc) return rc;
     if (n_ids < 1 || n_ids > kMaxIds)
         return set_error(MESHY_EINVAL, "%s: n_ids must be in [1, %d], got %lld", who, kMaxIds,
                          static_cast<long long>(n_ids));
+    if (max_polls < 0) return set_error(MESHY_EINVAL, "%s: negative max_polls", who);
     if (rows * T == 0) return MESHY_OK;
     if (!ids || !out) return set_error(MESHY_ENULL, "%s: ids and out are required", who);
     return launch_fwd(logits, rows, T, V, stride_b, stride_t, ids, static_cast<int>(n_ids), out, nullptr, lse,
-                      stream, who);
+                      stream, who, std::min(max_polls, kSplitPolls));
+}
+
+}  // namespace
+}  // namespace meshy
+
+extern "C" int meshy_logprob_entropy_fwd(const uint16_t* logits, int64_t rows, int64_t T, int64_t V,
+                                         int64_t stride_b, int64_t stride_t, const int64_t* labels,
+                                         float* logp, float* entropy, float* lse,
+                                         hipStream_t stream) {
+    return meshy::entropy_fwd(logits, rows, T, V, stride_b, stride_t, labels, logp, entropy, lse,
+                              meshy::kSplitPolls, stream, "meshy_logprob_entropy_fwd");
+}
+
+extern "C" int meshy_logprob_entropy_fwd_polls(const uint16_t* logits, int64_t rows, int64_t T, int64_t V,
+                                               int64_t stride_b, int64_t stride_t, const int64_t* labels,
+                                               float* logp, float* entropy, float* lse, int32_t max_polls,
+                                               hipStream_t stream) {
+    return meshy::entropy_fwd(logits, rows, T, V, stride_b, stride_t, labels, logp, entropy, lse, max_polls, stream,
+                              "meshy_logprob_entropy_fwd_polls");
+}
+
+extern "C" int meshy_gather_logprobs_fwd(const uint16_t* logits, int64_t rows, int64_t T, int64_t V,
+                                         int64_t stride_b, int64_t stride_t, const int64_t* ids,
+                                         int64_t n_ids, float* out, float* lse, hipStream_t stream) {
+    return meshy::gather_fwd(logits, rows, T, V, stride_b, stride_t, ids, n_ids, out, lse, meshy::kSplitPolls, stream,
+                             "meshy_gather_logprobs_fwd");
+}
+
+extern "C" int meshy_gather_logprobs_fwd_polls(const uint16_t* logits, int64_t rows, int64_t T, int64_t V,
+                                               int64_t stride_b, int64_t stride_t, const int64_t* ids,
+                                               int64_t n_ids, float* out, float* lse, int32_t max_polls,
+                                               hipStream_t stream) {
+    return meshy::gather_fwd(logits, rows, T, V, stride_b, stride_t, ids, n_ids, out, lse, max_polls, stream,
+                             "meshy_gather_logprobs_fwd_polls");
 }
 
 extern "C" size_t meshy_logprob_bwd_workspace_size(int64_t n_rows) {

@@ -86,6 +86,31 @@ def test_polls_that_run_out(n):
     _check(logits, labels, logp, ent)
 
 
+@pytest.mark.parametrize("n", [1, 16, 37, 127])
+@pytest.mark.parametrize("V", [49153, 151936])
+def test_outputs_do_not_depend_on_who_took_the_parts(n, V):
+    # max_polls = 0: the last part's workgroup does not look and takes every part.
+    lib, stream = _lib.load(), _lib.stream_of(torch.device("cuda:0"))
+    logits, labels = _logits(n, V, n + V + 1, offset=3)
+    ids = torch.randint(V, (1, n, 9), device="cuda")
+    shape = (logits.data_ptr(), 1, n, V, logits.stride(0), logits.stride(1))
+    results = []
+    for polls in (4000, 0, 1):
+        logp, ent, lse, lse_of_gather = torch.empty(4, 1, n, device="cuda").unbind()
+        out = torch.empty(1, n, 9, device="cuda")
+        _lib.check(lib.meshy_logprob_entropy_fwd_polls(*shape, labels.data_ptr(), logp.data_ptr(), ent.data_ptr(),
+                                                       lse.data_ptr(), polls, stream), "entropy")
+        _lib.check(lib.meshy_gather_logprobs_fwd_polls(*shape, ids.data_ptr(), 9, out.data_ptr(),
+                                                       lse_of_gather.data_ptr(), polls, stream), "gather")
+        results.append((logp, ent, lse, lse_of_gather, out))
+    _check(logits, labels, logp, ent)
+    torch.testing.assert_close(out.double(), _exact(logits, ids)[0], rtol=0, atol=LOGP_ATOL)
+    for other in results[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(results[0], other))
+    eager = logprobs_and_entropy(logits, labels, with_entropy=True)
+    assert torch.equal(eager[0], logp) and torch.equal(eager[1], ent)
+
+
 def test_calls_on_two_streams():
     logits, labels = _logits(37, 151936, 9)
     first = logprobs_and_entropy(logits, labels, with_entropy=True)
