@@ -54,8 +54,6 @@ __device__ __forceinline__ int dpp_i32(int v) {
     return __builtin_amdgcn_update_dpp(0, v, kCtrl, 0xF, 0xF, false);
 }
 constexpr int kDppRowRor1 = 0x121, kDppRowRor2 = 0x122, kDppRowRor4 = 0x124, kDppRowRor8 = 0x128;
-// Whole-wavefront shift: lane l takes lane l - 1's value, lane 0 gets 0.
-constexpr int kDppWaveShr1 = 0x138;
 
 template <int kCtrl>
 __device__ __forceinline__ float dpp_f32(float v) {
@@ -81,11 +79,17 @@ __device__ __forceinline__ double lane_f64(double v, int lane) {
     return __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi) << 32) | lo));
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
+// The sum over each 16-lane row, in every lane of the row.
+__device__ __forceinline__ float row16_sum(float v) {
     v += dpp_f32<kDppRowRor8>(v);
     v += dpp_f32<kDppRowRor4>(v);
     v += dpp_f32<kDppRowRor2>(v);
     v += dpp_f32<kDppRowRor1>(v);
+    return v;
+}
+
+__device__ __forceinline__ float wave_sum(float v) {
+    v = row16_sum(v);
     return (lane_f32(v, 0) + lane_f32(v, 16)) + (lane_f32(v, 32) + lane_f32(v, 48));
 }
 

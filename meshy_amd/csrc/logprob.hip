@@ -26,30 +26,44 @@
 namespace meshy {
 namespace {
 
-constexpr int kMaxIds = 256;  // gather ids per row (one thread each)
+constexpr int kMaxIds = 256;  // gather ids per row
 
-// thread 0: lse, entropy, and (with one id) the log-prob.
+// The log-prob of an id with logit zy.
 __device__ __forceinline__ float id_logp(int64_t y, float zy, float lse, int64_t V) {
     if (y == kIgnoreIndex) return 0.f;
     if (y < 0 || y >= V) return __builtin_nanf("");
     return zy - lse;
 }
 
-// Loads the row's gather id for thread `tid` (< n_ids) and its logit.
-__device__ __forceinline__ void load_id(const uint16_t* row, const int64_t* ids, int64_t r, int n_ids,
-                                        int64_t V, int64_t& y, float& zy) {
-    y = 0;
-    zy = 0.f;
-    const int tid = threadIdx.x;
-    if (ids && tid < n_ids) {
-        y = ids[r * n_ids + tid];
-        if (y >= 0 && y < V) zy = bf16_to_f32(row[y]);
+// The row's gather ids that a thread of NT takes (id tid + NT j in y[j]) and
+// their logits.
+template <int NT>
+struct RowIds {
+    static constexpr int kPer = (kMaxIds + NT - 1) / NT;
+    int64_t y[kPer];
+    float z[kPer];
+};
+
+template <int NT>
+__device__ __forceinline__ RowIds<NT> load_ids(const uint16_t* row, const int64_t* ids, int64_t r, int n_ids,
+                                               int64_t V) {
+    RowIds<NT> w;
+#pragma unroll
+    for (int j = 0; j < RowIds<NT>::kPer; ++j) {
+        const int k = threadIdx.x + j * NT;
+        w.y[j] = 0;
+        w.z[j] = 0.f;
+        if (ids && k < n_ids) {
+            w.y[j] = ids[r * n_ids + k];
+            if (w.y[j] >= 0 && w.y[j] < V) w.z[j] = bf16_to_f32(row[w.y[j]]);
+        }
     }
+    return w;
 }
 
 // Writes the row's outputs once block_merge has left (m, s, t) in thread 0.
 template <int NT>
-__device__ __forceinline__ void finish_row(int64_t r, float m, float s, float t, int64_t y, float zy,
+__device__ __forceinline__ void finish_row(int64_t r, float m, float s, float t, const RowIds<NT>& w,
                                            int64_t V, int n_ids, float* logp, float* ent, float* lse_out) {
     __shared__ float s_lse;
     if (threadIdx.x == 0) {
@@ -57,12 +71,16 @@ __device__ __forceinline__ void finish_row(int64_t r, float m, float s, float t,
         const float lse = fmaf(l2s, kLn2, m);
         if (lse_out) lse_out[r] = lse;
         if (ent) ent[r] = kLn2 * (l2s - t / s);
-        if (n_ids == 1 && logp) logp[r] = id_logp(y, zy, lse, V);
+        if (n_ids == 1 && logp) logp[r] = id_logp(w.y[0], w.z[0], lse, V);
         s_lse = lse;
     }
     if (n_ids > 1 && logp) {
         __syncthreads();
-        if (static_cast<int>(threadIdx.x) < n_ids) logp[r * n_ids + threadIdx.x] = id_logp(y, zy, s_lse, V);
+#pragma unroll
+        for (int j = 0; j < RowIds<NT>::kPer; ++j) {
+            const int k = threadIdx.x + j * NT;
+            if (k < n_ids) logp[r * n_ids + k] = id_logp(w.y[j], w.z[j], s_lse, V);
+        }
     }
 }
 
@@ -160,8 +178,8 @@ struct Split {
     int max_polls;
 };
 
-// Bound by the read of the logits.  NT threads per workgroup (fwd_threads), U
-// 16-byte loads in flight per thread per tile.  A lane's first tile sets its
+// Bound by the read of the logits.  NT threads per workgroup and U 16-byte loads
+// in flight per thread per tile (fwd_shape).  A lane's first tile sets its
 // running max; later tiles are accumulated against it (accumulate_at) and take
 // the tile max only when an element lies more than 44 above it.  The chunks left
 // after the full tiles form one predicated tile.
@@ -181,15 +199,14 @@ __global__ __launch_bounds__(NT) void k_lpe_fwd_vec(const uint16_t* __restrict__
                                                     const int64_t* __restrict__ ids, int n_ids,
                                                     float* __restrict__ logp, float* __restrict__ ent,
                                                     float* __restrict__ lse_out, Split sx) {
+    static_assert(NT >= kLineElems + 8, "a thread per element outside the chunks");
     const int part = kSplit ? static_cast<int>(blockIdx.x) / sx.n_rows : 0;
     const int64_t r = kSplit ? static_cast<int>(blockIdx.x) % sx.n_rows : static_cast<int64_t>(blockIdx.x);
     const bool last = !kSplit || part + 1 == sx.parts;
     const uint16_t* row = row_ptr(logits, r, T, stride_b, stride_t);
     const RowSpan sp = row_span(row, V);
     const int tid = threadIdx.x;
-    int64_t y;
-    float zy;
-    load_id(row, ids, r, n_ids, V, y, zy);
+    const RowIds<NT> w = load_ids<NT>(row, ids, r, n_ids, V);
     bool edge;
     const int64_t e = edge_element(sp, V, tid, edge);
     edge = edge && last;
@@ -236,10 +253,10 @@ __global__ __launch_bounds__(NT) void k_lpe_fwd_vec(const uint16_t* __restrict__
                     const int slot = part * sx.n_rows + static_cast<int>(r);
                     const float v[3] = {m, s, t};
 #pragma unroll
-                    for (int w = 0; w < 3; ++w)
-                        __hip_atomic_store(&slots[slot].w[w],
-                                           (static_cast<unsigned long long>(split_tag(sx.call, slot, w)) << 32) |
-                                               __float_as_uint(v[w]),
+                    for (int i = 0; i < 3; ++i)
+                        __hip_atomic_store(&slots[slot].w[i],
+                                           (static_cast<unsigned long long>(split_tag(sx.call, slot, i)) << 32) |
+                                               __float_as_uint(v[i]),
                                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 }
                 return;
@@ -270,7 +287,7 @@ __global__ __launch_bounds__(NT) void k_lpe_fwd_vec(const uint16_t* __restrict__
             p = p == part ? 0 : p + 1;
         }
     }
-    finish_row<NT>(r, m, s, t, y, zy, V, n_ids, logp, ent, lse_out);
+    finish_row<NT>(r, m, s, t, w, V, n_ids, logp, ent, lse_out);
 }
 
 // ---------------------------------------------------------------- backward
@@ -532,8 +549,9 @@ __global__ __launch_bounds__(NT) void k_lp_bwd_any(BwdArgs a) {
     }
 }
 
-// 16-byte loads in flight per thread per tile (4 are slower at every size).
-constexpr int kFwdUnroll = 8;
+// 16-byte loads in flight per thread per tile, for the rows that fill several
+// tiles and for the others (their last tile is predicated and rounds up).
+constexpr int kFwdUnroll = 8, kFwdShortUnroll = 2;
 constexpr int kBwdThreads = 256;
 constexpr int kBwdUnroll = 2;
 constexpr int64_t kBwdMinFlatV = 256;
@@ -553,18 +571,32 @@ int check_common(const void* logits, int64_t rows, int64_t T, int64_t V, int64_t
     return MESHY_OK;
 }
 
-// Threads of a workgroup that takes a whole row.  Up to 256 rows there is one
-// workgroup per CU at most, and a CU streams in proportion to its loads in
-// flight: 512 threads take 13.0 us for 37 undivided rows of 151936 logits and
-// 16.0 for 256, against 19.1 and 21.1 with 256 threads (1024 threads: 12.4 and
-// 16.3).  From 257 rows on, 256
-// threads spread the rows more evenly (512 rows: 27.4 against 28.1 us; 4096
-// rows of 50257: 65.6 against 72.2, where most of a row is the predicated last
-// tile of 4096 chunks).  Many rows of at least 3 full tiles of 512 threads
-// stream faster with those (4096 rows of 131072: 158.0 against 162.4 us; 16384
-// of 151936: 703 against 714; 4096 of 81920, 2.5 tiles: 102.2 against 103.5).
-int fwd_threads(int64_t n, int64_t V) {
-    return n <= 256 || (n >= 2048 && V >= 3 * 512 * kFwdUnroll * 8) ? 512 : 256;
+// Threads and loads per thread of a workgroup that takes a whole row.
+// Up to 256 rows there is one workgroup per CU at most, and a CU streams in
+// proportion to its loads in flight: 512 threads of 8 loads take 13.0 us for 37
+// undivided rows of 151936 logits, 256 threads 19.1.  From 2048 rows on, long
+// rows (3 full tiles and more) stream fastest with those too (16384 rows of
+// 151936: 703 us against 714 with 256 threads; 4096: 181 against 184 with 2
+// loads).  All others take the registers of 2 loads and 8 waves per SIMD, in
+// fewer threads where a short row would leave them idle, as long as the rows
+// still fill the CUs (128 threads: 16 workgroups per CU, 4096 in all):
+//   4096 rows of 65537 logits    512 x 2: 80 us   256 x 2: 82   256 x 8: 83
+//   4096 rows of 32768           512 x 2: 42      256 x 2: 43   256 x 8: 43
+//   4096 rows of 16384           256 x 2: 23      512 x 2: 24   256 x 8: 25
+//   1024 rows of 24576           512 x 2: 9.9     256 x 2: 10.3 256 x 8: 11.2
+//   16384 rows of 8192           128 x 2: 42      256 x 2: 44   256 x 8: 58
+//   2048 rows of 8192            256 x 2: 8.2     128 x 2: 9.2  256 x 8: 10.2
+//   131072 rows of 64            128 x 2: 84      256 x 2: 150  256 x 8: 190
+// Many gather ids of a row that is not the shortest want more threads (16384
+// rows of 4096, 200 ids: 38 us with 256, 42 with 128).
+struct FwdShape {
+    int threads, unroll;
+};
+
+FwdShape fwd_shape(int64_t n, int64_t V, int n_ids) {
+    if (n <= 256 || (n >= 2048 && V >= 3 * 512 * kFwdUnroll * 8)) return {512, kFwdUnroll};
+    if (V <= 1024 || (n_ids <= 128 && (V <= 4096 || (V <= 8192 && n >= 4096)))) return {128, kFwdShortUnroll};
+    return {V < 32768 && n > 1024 ? 256 : 512, kFwdShortUnroll};
 }
 
 // Workgroups per row.  One workgroup to a row is bound by its CU's exponentials
@@ -604,14 +636,15 @@ int launch_fwd(const uint16_t* logits, int64_t rows, int64_t T, int64_t V, int64
         return check_launch(who);
     }
     const dim3 grid(static_cast<unsigned>(n));
-    auto go = [&](auto kernel, int threads) {
-        hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, stream, logits, T, V, stride_b, stride_t, ids, n_ids, out,
-                           entropy, lse, Split{});
+    const FwdShape shape = fwd_shape(n, V, n_ids);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(shape.threads), 0, stream, logits, T, V, stride_b, stride_t, ids, n_ids,
+                           out, entropy, lse, Split{});
     };
-    if (fwd_threads(n, V) == 512)
-        go(k_lpe_fwd_vec<512, kFwdUnroll, false>, 512);
-    else
-        go(k_lpe_fwd_vec<256, kFwdUnroll, false>, 256);
+    if (shape.unroll == kFwdUnroll) go(k_lpe_fwd_vec<512, kFwdUnroll, false>);
+    else if (shape.threads == 512) go(k_lpe_fwd_vec<512, kFwdShortUnroll, false>);
+    else if (shape.threads == 256) go(k_lpe_fwd_vec<256, kFwdShortUnroll, false>);
+    else go(k_lpe_fwd_vec<128, kFwdShortUnroll, false>);
     return check_launch(who);
 }
 

@@ -26,19 +26,6 @@ constexpr int64_t kIgnoreIndex = -100;
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
-// Merges (m2, s2, t2) into (m, s, t); kEntropy = false leaves t untouched.
-template <bool kEntropy = true>
-__device__ __forceinline__ void merge(float& m, float& s, float& t, float m2, float s2, float t2) {
-    const float mn = fmaxf(m, m2);
-    const float d1 = (m - mn) * kLog2e;
-    const float d2 = (m2 - mn) * kLog2e;
-    const float a1 = fast_exp2(d1);
-    const float a2 = fast_exp2(d2);
-    if (kEntropy) t = a1 * fmaf(d1, s, t) + a2 * fmaf(d2, s2, t2);
-    s = a1 * s + a2 * s2;
-    m = mn;
-}
-
 // Moves the running max to at least `tm`, rescaling s and t.
 __device__ __forceinline__ void raise_max(float& m, float& s, float& t, float tm) {
     const float mn = fmaxf(m, tm);
@@ -188,43 +175,44 @@ __device__ __forceinline__ void accumulate_one(float z, bool ok, float& m, float
     t = fmaf(e, x, t);
 }
 
-// Merges each lane's triple with that of the lane kCtrl rotates to it.
-template <int kCtrl, bool kEntropy>
-__device__ __forceinline__ void merge_dpp(float& m, float& s, float& t) {
-    const float m2 = dpp_f32<kCtrl>(m);
-    const float s2 = dpp_f32<kCtrl>(s);
-    const float t2 = kEntropy ? dpp_f32<kCtrl>(t) : 0.f;
-    merge<kEntropy>(m, s, t, m2, s2, t2);
+// Moves the triple to the reference point top (>= m); kEntropy = false leaves
+// t untouched.
+template <bool kEntropy>
+__device__ __forceinline__ void rebase(float& m, float& s, float& t, float top) {
+    const float d = (m - top) * kLog2e;
+    const float a = fast_exp2(d);
+    if (kEntropy) t = a * fmaf(d, s, t);
+    s = a * s;
+    m = top;
 }
 
-// The merge over each 16-lane row through DPP rotations, valid in lane 0 of
-// the row.
+__device__ __forceinline__ float row16_max(float v) {
+    v = fmaxf(v, dpp_f32<kDppRowRor8>(v));
+    v = fmaxf(v, dpp_f32<kDppRowRor4>(v));
+    v = fmaxf(v, dpp_f32<kDppRowRor2>(v));
+    return fmaxf(v, dpp_f32<kDppRowRor1>(v));
+}
+
+// The merge over each 16-lane row, valid in every lane of the row.
 template <bool kEntropy>
 __device__ __forceinline__ void merge_rows16(float& m, float& s, float& t) {
-    merge_dpp<kDppRowRor8, kEntropy>(m, s, t);
-    merge_dpp<kDppRowRor4, kEntropy>(m, s, t);
-    merge_dpp<kDppRowRor2, kEntropy>(m, s, t);
-    merge_dpp<kDppRowRor1, kEntropy>(m, s, t);
+    rebase<kEntropy>(m, s, t, row16_max(m));
+    s = row16_sum(s);
+    if (kEntropy) t = row16_sum(t);
 }
 
-// Block-wide merge of the per-lane triples; the result lands in thread 0.
-// Rows of 16 lanes and then the waves' triples go through DPP rotations: with
-// 16 waves a chain of one merge per wave in thread 0 alone took longer than
-// the rest of the merge.
+// Block-wide merge of the per-lane triples; the result lands in wave 0.  The
+// maximum first, then every triple is moved to it and the sums add up, all
+// through DPP rotations: one exponential per wave.  (A tree of pairwise merges,
+// two exponentials each, is bound by the SIMDs' arithmetic for short rows:
+// 131072 rows of 64 logits took 262 us with one.)
 template <int NT, bool kEntropy = true>
 __device__ __forceinline__ void block_merge(float& m, float& s, float& t) {
-    merge_rows16<kEntropy>(m, s, t);
-    float mr[4], sr[4], tr[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        mr[r] = lane_f32(m, 16 * r);
-        sr[r] = lane_f32(s, 16 * r);
-        tr[r] = kEntropy ? lane_f32(t, 16 * r) : 0.f;
-    }
-    merge<kEntropy>(mr[0], sr[0], tr[0], mr[1], sr[1], tr[1]);
-    merge<kEntropy>(mr[2], sr[2], tr[2], mr[3], sr[3], tr[3]);
-    m = mr[0], s = sr[0], t = tr[0];
-    merge<kEntropy>(m, s, t, mr[2], sr[2], tr[2]);
+    const float top = row16_max(m);
+    rebase<kEntropy>(m, s, t, fmaxf(fmaxf(lane_f32(top, 0), lane_f32(top, 16)),
+                                    fmaxf(lane_f32(top, 32), lane_f32(top, 48))));
+    s = wave_sum(s);
+    if (kEntropy) t = wave_sum(t);
     if constexpr (NT > kWave) {
         constexpr int kWaves = NT / kWave;
         static_assert(kWaves <= 16, "the waves' triples are merged in one row of 16 lanes");

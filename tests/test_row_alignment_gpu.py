@@ -60,6 +60,23 @@ def test_forward_on_both_sides_of_the_workgroup_size_rule(dev, T, V):
     assert (ent[:, rows].cpu() - olp.chunk_entropy(z, dtype=torch.float64)).abs().max().item() <= TOL
 
 
+# Both sides of the bounds on rows, logits and ids that choose a workgroup's
+# threads and loads for short and middle rows.
+@pytest.mark.parametrize("T,V,K", [(257, 1024, 256), (257, 1025, 128), (257, 1025, 129), (257, 4097, 256), (4095, 8192, 9),
+                                   (4096, 8192, 200), (4096, 8193, 9), (1024, 20001, 9), (1025, 20001, 9), (1025, 32767, 9), (1025, 32768, 9), (257, 131073, 200)])
+def test_gather_on_both_sides_of_the_shape_rules(dev, T, V, K):
+    from meshy_amd import logprob, topk
+
+    g = torch.Generator(device=dev).manual_seed(T + V)
+    zd = torch.randn(1, T, V + 1, generator=g, device=dev, dtype=torch.bfloat16).mul_(2.0)[..., 1:]
+    ids = torch.randint(0, V, (1, T, K), generator=g, device=dev)
+    out, lp = topk.gather_logprobs(zd, ids), logprob.logprobs_and_entropy(zd, ids[..., K - 1])
+    rows = torch.cat([torch.arange(0, T, 97), torch.tensor([T - 1])]).to(dev)
+    ref = torch.log_softmax(zd[:, rows].double(), -1).gather(-1, ids[:, rows])
+    assert (out[:, rows] - ref).abs().max().item() <= TOL
+    assert (lp[:, rows] - ref[..., K - 1]).abs().max().item() <= TOL
+
+
 def _grad_ref(z, ids, g, lse):
     """float64 gradient of sum(g * (z[ids] - lse)) given the fp32 lse the kernel reads."""
     n, V = z.shape
