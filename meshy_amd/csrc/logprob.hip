@@ -29,10 +29,10 @@ namespace {
 constexpr int kMaxIds = 256;  // gather ids per row
 
 // The log-prob of an id with logit zy.
-__device__ __forceinline__ float id_logp(int64_t y, float zy, float lse, int64_t V) {
+__device__ __forceinline__ float id_logp(int64_t y, float zy, double lse, int64_t V) {
     if (y == kIgnoreIndex) return 0.f;
     if (y < 0 || y >= V) return __builtin_nanf("");
-    return zy - lse;
+    return static_cast<float>(zy - lse);
 }
 
 // The row's gather ids that a thread of NT takes (id tid + NT j in y[j]) and
@@ -61,16 +61,17 @@ __device__ __forceinline__ RowIds<NT> load_ids(const uint16_t* row, const int64_
     return w;
 }
 
-// Writes the row's outputs once block_merge has left (m, s, t) in thread 0.
+// Writes the row's outputs once block_merge has left (m, s, t) in thread 0,
+// which finishes them in double (lse_of).
 template <int NT>
 __device__ __forceinline__ void finish_row(int64_t r, float m, float s, float t, const RowIds<NT>& w,
                                            int64_t V, int n_ids, float* logp, float* ent, float* lse_out) {
-    __shared__ float s_lse;
+    __shared__ double s_lse;
     if (threadIdx.x == 0) {
-        const float l2s = __log2f(s);
-        const float lse = fmaf(l2s, kLn2, m);
-        if (lse_out) lse_out[r] = lse;
-        if (ent) ent[r] = kLn2 * (l2s - t / s);
+        const double l2s = log2_of(s);
+        const double lse = static_cast<double>(m) + l2s * kLn2Double;
+        if (lse_out) lse_out[r] = static_cast<float>(lse);
+        if (ent) ent[r] = static_cast<float>(kLn2Double * (l2s - static_cast<double>(t / s)));
         if (n_ids == 1 && logp) logp[r] = id_logp(w.y[0], w.z[0], lse, V);
         s_lse = lse;
     }

@@ -336,16 +336,6 @@ __device__ __forceinline__ bool topk_tile(v4u (&v)[G], OkF ok, int32_t col, bool
     return true;
 }
 
-// m + ln s in double, from the logarithm of s's mantissa (below 1 in magnitude).
-// In fp32 the log-sum-exp of a row of 150 thousand logits lies 3e-7 off by its
-// own rounding, and log2 of an s of 100 adds half of that: the log-probs of the
-// 8 best of 4096 rows of 151936 were 6.9e-8 off 64 bits, and are 2.7e-8 with it.
-__device__ __forceinline__ double lse_of(float m, float s) {
-    int e;
-    const float f = frexpf(s, &e);
-    return static_cast<double>(m) + (static_cast<double>(e) + static_cast<double>(__log2f(f))) * 0.6931471805599453;
-}
-
 // Bound by the read of the logits; NT threads per row as in the log-prob
 // forward.
 template <int NT, int U, int CAP>
