@@ -14,9 +14,9 @@
 // for the row's n_ids gather ids y_k.  No fp32 copy of the logits is made.
 //
 // Backward: grad[r, v] = sum_k g[r,k] onehot(y_k)[v] - G_r exp(z[r, v] - lse[r]),
-// G_r = sum_k g[r,k], written as bf16 in one pass over the flattened
-// [rows * V] gradient with a grid-stride loop: on MI355X that order writes 8 %
-// faster than one workgroup per row.
+// G_r = sum_k g[r,k], written as bf16 in one pass over the 16-byte chunks of the
+// flattened [rows * V] gradient, each taken once by a grid that covers them
+// (k_lp_bwd_flat); short rows go whole to waves or workgroups.
 #include <algorithm>
 #include <atomic>
 #include <type_traits>
@@ -295,7 +295,8 @@ __global__ __launch_bounds__(NT) void k_lpe_fwd_vec(const uint16_t* __restrict__
 
 struct BwdArgs {
     const uint16_t* logits;
-    int64_t T, V, stride_b, stride_t;
+    int64_t V, stride_b, stride_t;
+    uint32_t T;         // 0: every row lies stride_t after the one before
     int64_t row0;       // the launch's first row (a multiple of 8); the arrays below start at it
     int64_t n_elems;    // of the launch's gradient
     uint32_t n_chunks;  // ceil(n_elems / 8)
@@ -319,6 +320,12 @@ __device__ __forceinline__ bool row_id(const BwdArgs& a, int64_t r, int k, int64
     if (ignored) g = 0.f;
     if (ignored || bad) y = -1;
     return bad;
+}
+
+__device__ __forceinline__ const uint16_t* row_at(const BwdArgs& a, uint32_t r) {
+    if (a.T == 0) return a.logits + r * a.stride_t;
+    const uint32_t b = r / a.T;
+    return a.logits + b * a.stride_b + (r - b * a.T) * a.stride_t;
 }
 
 // What the pass needs of a row: ng = -G (NaN when an id is out of range),
@@ -399,33 +406,29 @@ __device__ __forceinline__ void locate(const BwdArgs& a, int64_t e, uint32_t& r,
     }
 }
 
-// The 8 logits of a chunk that one 16-byte load does not cover, element by
-// element (elements past the end repeat the last one).
-template <bool kContig>
-__device__ __forceinline__ v4u load_chunk_elements(const BwdArgs& a, int64_t e0) {
-    uint64_t half[2] = {0, 0};
-#pragma unroll 1
-    for (int k = 0; k < 8; ++k) {
-        const int64_t e = min(e0 + k, a.n_elems - 1);
-        uint64_t h;
-        if constexpr (kContig) {
-            h = a.logits[a.row0 * a.V + e];
-        } else {
-            uint32_t r;
-            int64_t pos;
-            locate(a, e, r, pos);
-            h = row_ptr(a.logits, a.row0 + r, a.T, a.stride_b, a.stride_t)[pos];
-        }
-        h <<= 16 * (k & 3);
-        half[0] |= k < 4 ? h : 0;
-        half[1] |= k < 4 ? 0 : h;
-    }
-    return v4u{static_cast<uint32_t>(half[0]), static_cast<uint32_t>(half[0] >> 32), static_cast<uint32_t>(half[1]),
-               static_cast<uint32_t>(half[1] >> 32)};
-}
-
 // 16 bytes at any element (the hardware's global loads need no alignment).
 typedef v4u v4u_any __attribute__((aligned(2)));
+
+__device__ __forceinline__ v4u load_any(const uint16_t* p) {
+    return __builtin_nontemporal_load(reinterpret_cast<const v4u_any*>(p));
+}
+
+// The last n (1 .. 7) of a's 8 elements, then b's first ones.
+__device__ __forceinline__ v4u join(const v4u& a, const v4u& b, int n) {
+    const uint64_t a0 = a.x | static_cast<uint64_t>(a.y) << 32, a1 = a.z | static_cast<uint64_t>(a.w) << 32;
+    const uint64_t b0 = b.x | static_cast<uint64_t>(b.y) << 32, b1 = b.z | static_cast<uint64_t>(b.w) << 32;
+    const int up = 16 * (n & 3), down = 64 - up;
+    uint64_t lo, hi;
+    if (n > 4) {
+        lo = up ? a0 >> down | a1 << up : a0;
+        hi = up ? a1 >> down | b0 << up : a1;
+    } else {
+        lo = up ? a1 >> down | b0 << up : a1;
+        hi = up ? b0 >> down | b1 << up : b0;
+    }
+    return v4u{static_cast<uint32_t>(lo), static_cast<uint32_t>(lo >> 32), static_cast<uint32_t>(hi),
+               static_cast<uint32_t>(hi >> 32)};
+}
 
 // A wave-uniform value moved to scalar registers.
 __device__ __forceinline__ int64_t uniform_i64(int64_t x) {
@@ -443,7 +446,9 @@ __device__ __forceinline__ int64_t uniform_i64(int64_t x) {
 // workgroups 1200; going from the last chunk to the first (towards what the
 // forward read last) changes nothing.  kContig: the logits are contiguous too,
 // so a chunk is 8 consecutive elements of both whatever V is; other logits are
-// read at their row's address.  Most waves' U groups lie in one row, whose
+// read at their row's address, and where a chunk holds a row's end, the row's
+// last 8 and the next row's first 8 are joined (16384 strided rows of 1000 logits
+// 14 us, 38 with such chunks read one by one).  Most waves' U groups lie in one row, whose
 // factors and ids are then wave-uniform: the wave reads them itself while its
 // logits are in flight, which costs less than the two passes over the rows
 // (factors before, one-hot terms after) that it replaces.  Waves that hold a
@@ -460,28 +465,46 @@ __global__ __launch_bounds__(NT) void k_lp_bwd_flat(BwdArgs a) {
     locate(a, e0, r, lo);
     r = __builtin_amdgcn_readfirstlane(r);
     lo = uniform_i64(lo);
-    const uint16_t* row = row_ptr(a.logits, a.row0 + r, a.T, a.stride_b, a.stride_t);
-    // Lanes past the end repeat the last whole chunk; a chunk that no one load
-    // covers is read again below.
+    const uint16_t* row = row_at(a, static_cast<uint32_t>(a.row0) + r);
+    // Lanes past the end repeat the last chunk.  A chunk whose 8 logits do not
+    // lie together (`part` of them end a row, or the tensor) is read below.
     v4u v[U];
+    const uint16_t* src[U];
+    int part[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-        const int64_t c = min<int64_t>(c0 + u * kWave + lane, last);
+        const int64_t e = min<int64_t>(c0 + u * kWave + lane, last) * 8;
+        part[u] = 0;
         if constexpr (kContig) {
-            const int64_t whole = c * 8 + 8 <= a.n_elems ? c : 0;
-            v[u] = __builtin_nontemporal_load(reinterpret_cast<const v4u*>(a.logits + a.row0 * a.V) + whole);
+            src[u] = a.logits + a.row0 * a.V + e;
+            if (e + 8 > a.n_elems) part[u] = static_cast<int>(a.n_elems - e);
         } else {
-            const int64_t p = lo + (c - c0) * 8;
-            v[u] = __builtin_nontemporal_load(reinterpret_cast<const v4u_any*>(row + (p + 8 <= a.V ? p : 0)));
+            uint32_t er = r;
+            int64_t pos = lo + (e - e0);
+            src[u] = row + pos;
+            if (pos + 8 > a.V) {
+                locate(a, e, er, pos);
+                src[u] = row_at(a, static_cast<uint32_t>(a.row0) + er) + pos;
+                if (pos + 8 > a.V) part[u] = static_cast<int>(a.V - pos);
+            }
         }
+        if (part[u]) src[u] -= 8 - part[u];
+        v[u] = load_any(src[u]);
     }
     const BwdRow<NB> w0 = bwd_row<NB>(a, r);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         const int64_t c = static_cast<int64_t>(c0) + u * kWave + lane;
         const int64_t e = c * 8;
-        if (kContig ? e + 8 > a.n_elems : lo + (e - e0) + 8 > a.V) {
-            if (c <= last) v[u] = load_chunk_elements<kContig>(a, e);
+        if (part[u]) {
+            v4u next{0, 0, 0, 0};
+            if constexpr (!kContig) {  // the next row's first logits
+                uint32_t er;
+                int64_t pos;
+                locate(a, min(c, last) * 8, er, pos);
+                if ((er + 1) * a.V < a.n_elems) next = load_any(row_at(a, static_cast<uint32_t>(a.row0) + er + 1));
+            }
+            v[u] = join(v[u], next, part[u]);
         }
         float z[8], q[8];
         const v4u vv[1] = {v[u]};
@@ -516,13 +539,127 @@ __global__ __launch_bounds__(NT) void k_lp_bwd_flat(BwdArgs a) {
     }
 }
 
-// One workgroup per row, an element per thread at a time: short rows, and
-// gradients that are not 16-byte aligned.  The one-hot positions are written
+// Orders the wave's memory operations before and after it across its lanes.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
+// Short rows: each wave takes R rows (a power of two, 8 to 64), whose gradient is
+// a whole number of 16-byte chunks of its own.  The lanes first read the rows'
+// factors (64 / R of them to a row's ids) into LDS, then take the chunks, each
+// with the factors of its row or rows.  One id per row is added in registers;
+// several are written again after the chunks, each with the gradients of every
+// id equal to its own.  inv = floor(2^32 / V) + 1: the rows' R V elements are few
+// enough for the row of one to be the high half of its product with inv.
+template <int NT, bool kOneId, bool kContig>
+__global__ __launch_bounds__(NT) void k_lp_bwd_short(BwdArgs a, uint32_t n_rows, int R, uint32_t inv) {
+    __shared__ float s_ng[NT / kWave][kWave], s_nl[NT / kWave][kWave], s_g[NT / kWave][kWave];
+    __shared__ int s_y[NT / kWave][kWave];
+    const int lane = threadIdx.x % kWave;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int64_t first = (static_cast<int64_t>(blockIdx.x) * (NT / kWave) + wid) * R;
+    if (first >= n_rows) return;
+    const uint32_t r0 = static_cast<uint32_t>(first);
+    const int rows = min(R, static_cast<int>(n_rows - r0));
+    const int V = static_cast<int>(a.V);
+    float *ng = s_ng[wid], *nl = s_nl[wid], *sg = s_g[wid];
+    int* sy = s_y[wid];
+    {
+        const int rl = lane & (R - 1);
+        const bool in = rl < rows;
+        float G = 0.f, g = 0.f;
+        int64_t y = -1;
+#pragma unroll 4
+        for (int k = lane / R; in && k < a.n_ids; k += kWave / R) {
+            const bool bad = row_id(a, r0 + rl, k, y, g);
+            G += bad ? __builtin_nanf("") : g;
+        }
+        for (int off = R; off < kWave; off <<= 1) G += __shfl_xor(G, off, kWave);
+        if (lane < R) {
+            ng[rl] = -G;
+            nl[rl] = in ? -a.lse[r0 + rl] * kLog2e : 0.f;
+            if (kOneId) {
+                sy[rl] = static_cast<int>(y);
+                sg[rl] = g;
+            }
+        }
+    }
+    wave_sync();
+    const int64_t base = r0 * a.V;  // the wave's first element (a multiple of 8)
+    const int n_el = rows * V;
+    for (int e = 8 * lane; e < n_el; e += 8 * kWave) {
+        int rl = static_cast<int>(__umulhi(static_cast<uint32_t>(e), inv));
+        int col = e - rl * V;
+        const bool whole = e + 8 <= n_el;  // else the tensor's end
+        float z[8];
+        if (kContig || col + 8 <= V) {
+            const uint16_t* src = kContig ? a.logits + base + e : row_at(a, r0 + rl) + col;
+            const v4u v[1] = {whole ? load_any(src) : join(load_any(src - (8 - (n_el - e))), v4u{0, 0, 0, 0}, n_el - e)};
+            unpack(v, z);
+        } else {
+            uint32_t h[8];
+            int er = rl, ec = col;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                if (ec == V) ec = 0, er = min(er + 1, rows - 1);
+                h[k] = row_at(a, r0 + er)[ec++];
+            }
+#pragma unroll
+            for (int k = 0; k < 8; ++k) z[k] = bf16_to_f32(static_cast<uint16_t>(h[k]));
+        }
+        float q[8];
+        if (col + 8 <= V) {
+            const float n = ng[rl], l = nl[rl];
+            const int d = kOneId ? sy[rl] - col : 0;  // below 0 without an id
+            const float g = kOneId ? sg[rl] : 0.f;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                q[k] = n * fast_exp2(fmaf(z[k], kLog2e, l));
+                if (kOneId) q[k] += d == k ? g : 0.f;
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                if (col == V) col = 0, rl = min(rl + 1, rows - 1);
+                q[k] = ng[rl] * fast_exp2(fmaf(z[k], kLog2e, nl[rl]));
+                if (kOneId) q[k] += sy[rl] == col ? sg[rl] : 0.f;
+                ++col;
+            }
+        }
+        uint16_t* out = a.out + base + e;
+        if (whole) {
+            const v4u o{pack_bf16x2(q[0], q[1]), pack_bf16x2(q[2], q[3]), pack_bf16x2(q[4], q[5]),
+                        pack_bf16x2(q[6], q[7])};
+            *reinterpret_cast<v4u*>(out) = o;
+        } else {
+            for (int k = 0; e + k < n_el; ++k) out[k] = bf16_bits(q[k]);
+        }
+    }
+    if constexpr (!kOneId) {
+        wave_sync();  // the chunks are written
+        for (int i = lane; i < rows * a.n_ids; i += kWave) {
+            const int rl = i / a.n_ids;
+            const int64_t id0 = static_cast<int64_t>(r0 + rl) * a.n_ids;
+            const int64_t y = a.ids[id0 + i - rl * a.n_ids];
+            const float n = ng[rl];
+            if (y < 0 || y >= V || isnan(n)) continue;  // ignored, or a row of NaN
+            float q = n * fast_exp2(fmaf(bf16_to_f32(row_at(a, r0 + rl)[y]), kLog2e, nl[rl]));
+            for (int k = 0; k < a.n_ids; ++k) q += a.ids[id0 + k] == y ? a.grad_logp[id0 + k] : 0.f;
+            a.out[base + rl * V + y] = bf16_bits(q);
+        }
+    }
+}
+
+// One workgroup per row, an element per thread at a time: short rows with many
+// ids (kBwdShortV), gradients that are not 16-byte aligned, and tensors of one
+// logit per row or fewer than 8 in all.  The one-hot positions are written
 // again after the row, each with the gradients of every id equal to its own.
 template <int NT, int NB>
 __global__ __launch_bounds__(NT) void k_lp_bwd_any(BwdArgs a) {
     const int64_t r = blockIdx.x;
-    const uint16_t* row = row_ptr(a.logits, r, a.T, a.stride_b, a.stride_t);
+    const uint16_t* row = row_at(a, static_cast<uint32_t>(r));
     uint16_t* grow = a.out + r * a.V;
     const BwdRow<NB> w = bwd_row<NB>(a, r);
     auto term = [&](int64_t e) { return w.ng * fast_exp2(fmaf(bf16_to_f32(row[e]), kLog2e, w.nl)); };
@@ -555,7 +692,21 @@ __global__ __launch_bounds__(NT) void k_lp_bwd_any(BwdArgs a) {
 constexpr int kFwdUnroll = 8, kFwdShortUnroll = 2;
 constexpr int kBwdThreads = 256;
 constexpr int kBwdUnroll = 2;
-constexpr int64_t kBwdMinFlatV = 256;
+// Below this a wave of the flat pass holds several rows and waits for the
+// factors of one after the other: with more than one id, rows go whole to waves
+// if they are many and their ids few, else to workgroups, whose threads add up
+// a row's ids from LDS.  In us (before: three launches through a workspace):
+//   rows x logits, ids     flat    waves   workgroups   before
+//   131072 x 64, 1                 8.3     43           17
+//   65536 x 264, 1         20      15                   20
+//   65536 x 264, 9         41      31                   39
+//   65536 x 200, 16                31      61           44
+//   65536 x 200, 64                216     88           256
+//   8192 x 256, 9          10.8    8.3     7.3          12.4
+//   1000 x 256, 64         41      77      5.7          34
+//   65536 x 512, 9         38      45      70           55
+// One id: the flat pass takes rows from half this length on.
+constexpr int64_t kBwdShortV = 512;
 constexpr int64_t kBwdMaxElems = int64_t{1} << 33;  // of one launch: 32-bit chunk indices
 
 // Shape checks; an empty call (rows * T == 0) accepts NULL arrays, as an
@@ -665,7 +816,8 @@ int launch_bwd(const uint16_t* logits, int64_t rows, int64_t T, int64_t V, int64
     const int64_t n = rows * T;
     BwdArgs a{};
     a.logits = logits;
-    a.T = T, a.V = V, a.stride_b = stride_b, a.stride_t = stride_t;
+    a.T = rows == 1 || stride_b == T * stride_t ? 0 : static_cast<uint32_t>(T);
+    a.V = V, a.stride_b = stride_b, a.stride_t = stride_t;
     a.inv_v = 1.0 / static_cast<double>(V);
     a.ids = ids, a.lse = lse, a.grad_logp = grad_out;
     a.out = grad_logits;
@@ -678,11 +830,28 @@ int launch_bwd(const uint16_t* logits, int64_t rows, int64_t T, int64_t V, int64
         else go(std::integral_constant<int, kMaxIds / kWave>());
     };
     int rc;
-    const bool contiguous = stride_t == V && (rows == 1 || stride_b == T * V) &&
-                            reinterpret_cast<uintptr_t>(logits) % 16 == 0;
-    // A wave takes the rows that it holds in turn: at 2 rows per group of 512
-    // elements that is as fast as one workgroup per row with 2-byte accesses.
-    if (V >= kBwdMinFlatV && reinterpret_cast<uintptr_t>(grad_logits) % 16 == 0) {
+    const bool contiguous = stride_t == V && a.T == 0;
+    const bool aligned = reinterpret_cast<uintptr_t>(grad_logits) % 16 == 0;
+    const bool flat = V >= kBwdShortV || (V >= kBwdShortV / 2 && n_ids == 1);
+    const bool by_waves = V >= 2 && n * V >= 8 && (n_ids == 1 || (n_ids <= 16 && n > 8192));
+    if (aligned && !flat && by_waves) {
+        int R = 8;  // rows of a wave: about 1024 elements, if there are rows for 8 waves per CU
+        while (R < kWave && R * V < 1024 && n >= 2 * R * 2048) R *= 2;
+        const dim3 blocks(static_cast<unsigned>(ceil_div(n, R * (kBwdThreads / kWave))));
+        const uint32_t inv = static_cast<uint32_t>((int64_t{1} << 32) / V + 1);
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, blocks, dim3(kBwdThreads), 0, stream, a, static_cast<uint32_t>(n), R, inv);
+        };
+        if (n_ids == 1) {
+            if (contiguous) go(k_lp_bwd_short<kBwdThreads, true, true>);
+            else go(k_lp_bwd_short<kBwdThreads, true, false>);
+        } else {
+            if (contiguous) go(k_lp_bwd_short<kBwdThreads, false, true>);
+            else go(k_lp_bwd_short<kBwdThreads, false, false>);
+        }
+        return check_launch(who);
+    }
+    if (aligned && flat) {
         const int64_t step = std::max<int64_t>(8, kBwdMaxElems / V / 8 * 8);
         for (int64_t r0 = 0; r0 < n; r0 += step) {
             a.row0 = r0;
