@@ -373,6 +373,12 @@ int meshy_gather_logprobs_bwd(const uint16_t* logits, int64_t rows, int64_t T, i
                               int64_t n_ids, const float* lse, const float* grad_out,
                               uint16_t* grad_logits, void* workspace, size_t workspace_bytes,
                               hipStream_t stream);
+/* meshy_gather_logprobs_bwd (meshy_logprob_bwd with n_ids = 1) without the
+ * workspace argument, for any number of rows. */
+int meshy_gather_logprobs_bwd_noalloc(const uint16_t* logits, int64_t rows, int64_t T, int64_t V,
+                                      int64_t stride_b, int64_t stride_t, const int64_t* ids,
+                                      int64_t n_ids, const float* lse, const float* grad_out,
+                                      uint16_t* grad_logits, hipStream_t stream);
 
 /* ------------------------------------------------------------------------
  * Teacher Top-K with log-probabilities (device), bf16 logits.

@@ -292,6 +292,11 @@ SIGNATURES = {
         [c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64, c_void_p, c_void_p, c_void_p,
          c_void_p, c_void_p],
     ),
+    "meshy_gather_logprobs_bwd_noalloc": (
+        c_int,
+        [c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64, c_void_p, c_int64, c_void_p,
+         c_void_p, c_void_p, c_void_p],
+    ),
     "meshy_gather_logprobs_fwd": (
         c_int,
         [c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64, c_void_p, c_int64, c_void_p,

@@ -991,6 +991,25 @@ extern "C" int meshy_logprob_bwd_noalloc(const uint16_t* logits, int64_t rows, i
     return launch_bwd(logits, rows, T, V, stride_b, stride_t, labels, 1, lse, grad_logp, grad_logits, stream, who);
 }
 
+namespace meshy {
+namespace {
+
+int check_gather_bwd(const uint16_t* logits, int64_t rows, int64_t T, int64_t V, int64_t stride_b, int64_t stride_t,
+                     const int64_t* ids, int64_t n_ids, const float* lse, const float* grad_out,
+                     const uint16_t* grad_logits, const char* who) {
+    int rc = check_common(logits, rows, T, V, stride_b, stride_t, who);
+    if (rc) return rc;
+    if (n_ids < 1 || n_ids > kMaxIds)
+        return set_error(MESHY_EINVAL, "%s: n_ids must be in [1, %d], got %lld", who, kMaxIds,
+                         static_cast<long long>(n_ids));
+    if (rows * T > 0 && (!ids || !lse || !grad_out || !grad_logits))
+        return set_error(MESHY_ENULL, "%s: ids, lse, grad_out and grad_logits are required", who);
+    return MESHY_OK;
+}
+
+}  // namespace
+}  // namespace meshy
+
 extern "C" int meshy_gather_logprobs_bwd(const uint16_t* logits, int64_t rows, int64_t T, int64_t V,
                                          int64_t stride_b, int64_t stride_t, const int64_t* ids,
                                          int64_t n_ids, const float* lse, const float* grad_out,
@@ -999,15 +1018,23 @@ extern "C" int meshy_gather_logprobs_bwd(const uint16_t* logits, int64_t rows, i
     using namespace meshy;
     clear_error();
     const char* who = "meshy_gather_logprobs_bwd";
-    int rc = check_common(logits, rows, T, V, stride_b, stride_t, who);
-    if (rc) return rc;
-    if (n_ids < 1 || n_ids > kMaxIds)
-        return set_error(MESHY_EINVAL, "%s: n_ids must be in [1, %d], got %lld", who, kMaxIds,
-                         static_cast<long long>(n_ids));
-    if (rows * T == 0) return MESHY_OK;
-    if (!ids || !lse || !grad_out || !grad_logits)
-        return set_error(MESHY_ENULL, "%s: ids, lse, grad_out and grad_logits are required", who);
+    int rc = check_gather_bwd(logits, rows, T, V, stride_b, stride_t, ids, n_ids, lse, grad_out, grad_logits, who);
+    if (rc || rows * T == 0) return rc;
     if ((rc = check_bwd_ws(rows * T, workspace, workspace_bytes, who))) return rc;
+    return launch_bwd(logits, rows, T, V, stride_b, stride_t, ids, static_cast<int>(n_ids), lse, grad_out,
+                      grad_logits, stream, who);
+}
+
+extern "C" int meshy_gather_logprobs_bwd_noalloc(const uint16_t* logits, int64_t rows, int64_t T, int64_t V,
+                                                 int64_t stride_b, int64_t stride_t, const int64_t* ids,
+                                                 int64_t n_ids, const float* lse, const float* grad_out,
+                                                 uint16_t* grad_logits, hipStream_t stream) {
+    using namespace meshy;
+    clear_error();
+    const char* who = "meshy_gather_logprobs_bwd_noalloc";
+    const int rc =
+        check_gather_bwd(logits, rows, T, V, stride_b, stride_t, ids, n_ids, lse, grad_out, grad_logits, who);
+    if (rc || rows * T == 0) return rc;
     return launch_bwd(logits, rows, T, V, stride_b, stride_t, ids, static_cast<int>(n_ids), lse, grad_out,
                       grad_logits, stream, who);
 }

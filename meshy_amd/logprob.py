@@ -6,7 +6,7 @@ to fp32, runs ``-cross_entropy`` on it, then upcasts ``entropy_chunk_size``
 slices again for ``logsumexp - sum(softmax * z)``.  Here one HIP kernel
 (``meshy_logprob_entropy_fwd``) streams each row of bf16 logits from HBM
 once and returns both values in fp32; under autograd the backward kernel
-(``meshy_logprob_bwd``) rebuilds ``softmax`` from the saved per-row
+(``meshy_gather_logprobs_bwd_noalloc``) rebuilds ``softmax`` from the saved per-row
 log-sum-exp instead of a checkpointed recompute.
 """
 
@@ -56,7 +56,8 @@ def _fwd(logits, labels, *, want_logp: bool, want_entropy: bool, want_lse: bool)
 
 
 def bwd_workspace(n_rows: int, device) -> torch.Tensor:
-    """Scratch of the logprob / gather backward: two floats per row."""
+    """The workspace that the C entries ``meshy_logprob_bwd`` and
+    ``meshy_gather_logprobs_bwd`` ask for (they do not touch it)."""
     nbytes = int(_lib.load().meshy_logprob_bwd_workspace_size(n_rows))
     return torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
 
@@ -83,14 +84,10 @@ class _FusedLogprob(torch.autograd.Function):
         rows, T, V = logits.shape
         grad = torch.empty(rows, T, V, dtype=logits.dtype, device=logits.device)
         g = grad_logp.float().contiguous()
-        lib = _lib.load()
-        ws = bwd_workspace(rows * T, logits.device)
-        rc = lib.meshy_logprob_bwd(
-            logits.data_ptr(), rows, T, V, logits.stride(0), logits.stride(1), labels.data_ptr(),
-            lse.data_ptr(), g.data_ptr(), grad.data_ptr(), ws.data_ptr(), ws.numel(),
-            _lib.stream_of(logits.device),
-        )
-        _lib.check(rc, "meshy_logprob_bwd")
+        rc = _lib.load().meshy_gather_logprobs_bwd_noalloc(
+            logits.data_ptr(), rows, T, V, logits.stride(0), logits.stride(1), labels.data_ptr(), 1,
+            lse.data_ptr(), g.data_ptr(), grad.data_ptr(), _lib.stream_of(logits.device))
+        _lib.check(rc, "meshy_gather_logprobs_bwd_noalloc")
         return grad, None, None
 
 

@@ -7,7 +7,7 @@ fp32 (topk_loss.py:26-31, 50-56) and recomputing the chunk in backward.  Here
 each function streams every row of bf16 logits from HBM once:
 
 * ``teacher_topk``     ``meshy_topk_logprobs`` (Top-K and log-sum-exp in one pass);
-* ``gather_logprobs``  ``meshy_gather_logprobs_fwd`` / ``_bwd`` (the fused
+* ``gather_logprobs``  ``meshy_gather_logprobs_fwd`` / ``_bwd_noalloc`` (the fused
                        log-softmax gather of the PPO path with K ids per row);
 * ``forward_kl_topk``  ``meshy_forward_kl_topk`` / ``_bwd``.
 
@@ -19,7 +19,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from .logprob import _prep, bwd_workspace
+from .logprob import _prep
 
 
 def _dense(logits: torch.Tensor) -> torch.Tensor:
@@ -74,12 +74,10 @@ class _GatherLogprobs(torch.autograd.Function):
         K = ids.shape[-1]
         grad = torch.empty(rows, S, V, dtype=logits.dtype, device=logits.device)
         g = grad_out.float().contiguous()
-        ws = bwd_workspace(rows * S, logits.device)
-        rc = _lib.load().meshy_gather_logprobs_bwd(
+        rc = _lib.load().meshy_gather_logprobs_bwd_noalloc(
             logits.data_ptr(), rows, S, V, logits.stride(0), logits.stride(1), ids.data_ptr(), K,
-            lse.data_ptr(), g.data_ptr(), grad.data_ptr(), ws.data_ptr(), ws.numel(),
-            _lib.stream_of(logits.device))
-        _lib.check(rc, "meshy_gather_logprobs_bwd")
+            lse.data_ptr(), g.data_ptr(), grad.data_ptr(), _lib.stream_of(logits.device))
+        _lib.check(rc, "meshy_gather_logprobs_bwd_noalloc")
         return grad, None
 
 

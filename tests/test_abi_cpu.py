@@ -43,6 +43,10 @@ def _call(name, *args):
     ("meshy_logprob_bwd_noalloc", (FAKE, 1, 4, 8, 32, 8, FAKE, FAKE, FAKE, None, None), ENULL, "required"),
     ("meshy_gather_logprobs_bwd", (FAKE, 1, 4, 8, 32, 8, FAKE, 300, FAKE, FAKE, FAKE, FAKE, 4096, None), EINVAL,
      "n_ids"),
+    ("meshy_gather_logprobs_bwd_noalloc", (FAKE, 1, 4, 8, 32, 8, FAKE, 257, FAKE, FAKE, FAKE, None), EINVAL, "n_ids"),
+    ("meshy_gather_logprobs_bwd_noalloc", (FAKE, 1, 4, 8, 32, 8, None, 9, FAKE, FAKE, FAKE, None), ENULL, "required"),
+    ("meshy_logprob_entropy_fwd_polls", (FAKE, 1, 4, 8, 32, 8, FAKE, FAKE, None, None, -1, None), EINVAL, "max_polls"),
+    ("meshy_gather_logprobs_fwd_polls", (FAKE, 1, 4, 8, 32, 8, FAKE, 9, FAKE, None, -1, None), EINVAL, "max_polls"),
     # logits, rows, T, V, sb, st, k, ids, logprobs, lse, stream
     ("meshy_topk_logprobs", (FAKE, 1, 4, 100, 400, 100, 65, FAKE, FAKE, None, None), EINVAL, "k must be"),
     ("meshy_topk_logprobs", (FAKE, 1, 4, 5, 20, 5, 8, FAKE, FAKE, None, None), EINVAL, "k must be"),

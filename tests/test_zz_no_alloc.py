@@ -1,10 +1,11 @@
 """meshy_logprob_bwd_noalloc (the allocation-free backward) against
-meshy_logprob_bwd, both called through the C ABI.
+meshy_logprob_bwd and float64, both called through the C ABI.
 
-Both run the same kernels, the first with its per-row scratch in a static
-device array, the second in a caller workspace, so the bf16 gradients must be
-bitwise equal.  Two calls in a row, the second smaller, check that the array
-keeps nothing a later call depends on.
+Both are the same launch and touch no scratch, so the bf16 gradients must be
+bitwise equal, whatever was in the gradient before, over two calls in a row of
+which the second is smaller.  Sampled rows are compared with float64: bf16 rounds
+to 2^-9 relative, and the fp32 exponent of up to 16 adds less than 1e-5 of the
+row's gradient.
 """
 
 import pytest
@@ -62,3 +63,8 @@ def test_no_alloc_matches_workspace_entry_point_on_two_calls(dev):
         assert torch.equal(a.view(torch.int16), b.view(torch.int16))
         assert torch.isfinite(a.float()).all()
         assert (a[0, 0].float() == 0).all()  # the ignored label's row
+        for t in (1, T // 2, T - 1):
+            want = -gl[-1, t].double() * (z[-1, t].double() - lse[-1, t].double()).exp()
+            want[y[-1, t]] += gl[-1, t].double()
+            err = (a[-1, t].double() - want).abs()
+            assert (err <= 2.0 ** -8 * want.abs() + 1e-5 * gl[-1, t].abs()).all()
