@@ -8,6 +8,10 @@
 //     t = sum exp(z - m) * (z - m) * log2(e)   (only for the entropy)
 // updated once per register tile: the tile max first, then one exp2 per
 // element.  lse = m + ln s and H = ln 2 * (log2 s - t / s).
+// The exponent of an element is one fma, z log2(e) + ref(m), whose ref(m) is
+// -m log2(e) rounded: every term of s is off by the same 2^(m log2(e) + ref(m)),
+// which moves from one reference to the next by the difference of the two ref's
+// and is taken out at the end (ref_error).
 #pragma once
 
 #include <hip/hip_bf16.h>
@@ -26,10 +30,32 @@ constexpr int64_t kIgnoreIndex = -100;
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
+// (Its product must not be fused with what it is added to: the same ref(m) has
+// to come out everywhere.)
+__device__ __forceinline__ float ref(float m) {
+#pragma clang fp contract(off)
+    return -m * kLog2e;
+}
+
+// log2 of the factor that every term of s carries.
+__device__ __forceinline__ float ref_error(float m) { return fmaf(m, kLog2e, ref(m)); }
+
+__device__ __forceinline__ float row16_max(float v) {
+    v = fmaxf(v, dpp_f32<kDppRowRor8>(v));
+    v = fmaxf(v, dpp_f32<kDppRowRor4>(v));
+    v = fmaxf(v, dpp_f32<kDppRowRor2>(v));
+    return fmaxf(v, dpp_f32<kDppRowRor1>(v));
+}
+
+__device__ __forceinline__ float wave_max(float v) {
+    v = row16_max(v);
+    return fmaxf(fmaxf(lane_f32(v, 0), lane_f32(v, 16)), fmaxf(lane_f32(v, 32), lane_f32(v, 48)));
+}
+
 // Moves the running max to at least `tm`, rescaling s and t.
 __device__ __forceinline__ void raise_max(float& m, float& s, float& t, float tm) {
     const float mn = fmaxf(m, tm);
-    const float d = (m - mn) * kLog2e;
+    const float d = ref(mn) - ref(m);
     const float a = fast_exp2(d);
     t = a * fmaf(d, s, t);
     s = a * s;
@@ -64,7 +90,7 @@ __device__ __forceinline__ float tile_max(const float (&z)[K]) {
 template <bool kEntropy, int K>
 __device__ __forceinline__ void accumulate(const float (&z)[K], float tm, float& m, float& s, float& t) {
     raise_max(m, s, t, tm);
-    const float nm = -m * kLog2e;
+    const float nm = ref(m);
     float s0 = 0.f, s1 = 0.f, t0 = 0.f, t1 = 0.f;
 #pragma unroll
     for (int i = 0; i < K; i += 2) {
@@ -88,17 +114,28 @@ __device__ __forceinline__ void accumulate(const float (&z)[K], float& m, float&
     accumulate<kEntropy>(z, tile_max(z), m, s, t);
 }
 
-// Accumulates a full tile against the running max m as it stands, without a
-// tile max.  Any reference point gives the same lse and entropy (s and t are
-// both relative to m), so this is exact as long as the sums stay finite: it
-// is taken only when the tile's sum is at most 2^64, i.e. no element exceeds
-// m by more than 64 / log2(e) = 44.4.  Otherwise (and for NaN or infinite
-// inputs) it returns false with (s, t) untouched, and the caller accumulates
-// the tile with its max.  Saves the tile max and the rescale of every tile
-// after a lane's first.
+// A lane's first tile: its reference is the wave's maximum, which later tiles
+// rarely exceed by much.
+template <bool kEntropy, int K>
+__device__ __forceinline__ void accumulate_first(const float (&z)[K], float& m, float& s, float& t) {
+    accumulate<kEntropy>(z, wave_max(tile_max(z)), m, s, t);
+}
+
+// Accumulates a full tile against the running reference m as it stands, without
+// a tile max.  Any reference gives the same lse and entropy (s and t are both
+// relative to m), but the exponent of an element d above it, and t, are rounded
+// at the size of d log2(e): this is taken only when the tile's sum is at most
+// 2^12, i.e. no element exceeds m by more than 12 / log2(e) = 8.3.  Otherwise
+// (and for NaN or infinite inputs) it returns false with (s, t) untouched, and
+// the caller accumulates the tile with its max.  (With 2^64, a logit of 16 to 40
+// among N(0, 1/4) left errors of 4e-6 in its log-prob and 1.3e-5 in the entropy;
+// now below 7e-7.)  Saves the tile max and the rescale of every tile after a
+// lane's first.
+constexpr float kMaxTileSum = 0x1p12f;
+
 template <bool kEntropy, int U>
 __device__ __forceinline__ bool accumulate_at(const v4u (&v)[U], float m, float& s, float& t) {
-    const float nm = -m * kLog2e;
+    const float nm = ref(m);
     float s0 = 0.f, s1 = 0.f, t0 = 0.f, t1 = 0.f;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -120,7 +157,7 @@ __device__ __forceinline__ bool accumulate_at(const v4u (&v)[U], float m, float&
     // Both sums are formed before the test and kept or dropped by a select:
     // a branch around the t update would keep every exp of the tile live.
     const float st = s0 + s1;
-    const bool ok = st <= 0x1p64f;
+    const bool ok = st <= kMaxTileSum;
     s = ok ? s + st : s;
     if (kEntropy) t = ok ? t + (t0 + t1) : t;
     return ok;
@@ -136,7 +173,7 @@ __device__ __forceinline__ void accumulate_masked(float (&z)[G * 8], const bool 
 #pragma unroll
         for (int k = 0; k < 8; ++k) z[8 * g + k] = ok[g] ? z[8 * g + k] : kInit;
     raise_max(m, s, t, tile_max(z));
-    const float nm = -m * kLog2e;
+    const float nm = ref(m);
     float s0 = 0.f, t0 = 0.f;
 #pragma unroll
     for (int g = 0; g < G; ++g) {
@@ -169,7 +206,7 @@ __device__ __forceinline__ void load_tail(const v4u* base, int64_t rem, int tid,
 __device__ __forceinline__ void accumulate_one(float z, bool ok, float& m, float& s, float& t) {
     if (!ok) return;
     raise_max(m, s, t, z);
-    const float x = (z - m) * kLog2e;
+    const float x = fmaf(z, kLog2e, ref(m));
     const float e = fast_exp2(x);
     s += e;
     t = fmaf(e, x, t);
@@ -179,18 +216,11 @@ __device__ __forceinline__ void accumulate_one(float z, bool ok, float& m, float
 // t untouched.
 template <bool kEntropy>
 __device__ __forceinline__ void rebase(float& m, float& s, float& t, float top) {
-    const float d = (m - top) * kLog2e;
+    const float d = ref(top) - ref(m);
     const float a = fast_exp2(d);
     if (kEntropy) t = a * fmaf(d, s, t);
     s = a * s;
     m = top;
-}
-
-__device__ __forceinline__ float row16_max(float v) {
-    v = fmaxf(v, dpp_f32<kDppRowRor8>(v));
-    v = fmaxf(v, dpp_f32<kDppRowRor4>(v));
-    v = fmaxf(v, dpp_f32<kDppRowRor2>(v));
-    return fmaxf(v, dpp_f32<kDppRowRor1>(v));
 }
 
 // The merge over each 16-lane row, valid in every lane of the row.
@@ -208,9 +238,7 @@ __device__ __forceinline__ void merge_rows16(float& m, float& s, float& t) {
 // 131072 rows of 64 logits took 262 us with one.)
 template <int NT, bool kEntropy = true>
 __device__ __forceinline__ void block_merge(float& m, float& s, float& t) {
-    const float top = row16_max(m);
-    rebase<kEntropy>(m, s, t, fmaxf(fmaxf(lane_f32(top, 0), lane_f32(top, 16)),
-                                    fmaxf(lane_f32(top, 32), lane_f32(top, 48))));
+    rebase<kEntropy>(m, s, t, wave_max(m));
     s = wave_sum(s);
     if (kEntropy) t = wave_sum(t);
     if constexpr (NT > kWave) {
@@ -235,21 +263,47 @@ __device__ __forceinline__ void block_merge(float& m, float& s, float& t) {
     }
 }
 
-constexpr double kLn2Double = 0.6931471805599453;
+// m + ln s as hi + lo in fp32, |lo| < 1, good to a few 2^-24: s = f 2^e with f in
+// [1, 2), so that a sum of 1 (one logit has all the weight) gives m itself, and
+// e ln 2 is split so that its high part is exact.  Rounded to one fp32, the
+// log-sum-exp of a row of 150 thousand logits lies 3e-7 off, as much as
+// everything else together.
+struct Lse {
+    float hi, lo;
+};
 
-// log2 s in double, from the logarithm of s's mantissa (below 1 in magnitude).
-__device__ __forceinline__ double log2_of(float s) {
-    int e;
-    const float f = frexpf(s, &e);
-    return static_cast<double>(e) + static_cast<double>(__log2f(f));
+constexpr float kLn2High = 2839.f / 4096.f;
+constexpr float kLn2Low = static_cast<float>(0.6931471805599453 - 2839.0 / 4096.0);
+
+// a + b = sum + err exactly, as long as sum is finite.
+__device__ __forceinline__ float add_with_error(float a, float b, float& err) {
+    const float sum = a + b;
+    const float bb = sum - a;
+    err = (a - (sum - bb)) + (b - bb);
+    return sum;
 }
 
-// m + ln s in double.  In fp32 the log-sum-exp of a row of 150 thousand logits
-// lies 3e-7 off by its own rounding, and log2 of an s of 100 adds half of that:
-// the log-probs of the 8 best of 4096 rows of 151936 were 6.9e-8 off 64 bits,
-// and are 2.7e-8 with it.
-__device__ __forceinline__ double lse_of(float m, float s) {
-    return static_cast<double>(m) + log2_of(s) * kLn2Double;
+// ln s as high + low, the high part exact.
+__device__ __forceinline__ Lse ln_of(float s) {
+    int e;
+    const float f = 2.f * frexpf(s, &e);
+    const float ef = static_cast<float>(e - 1);
+    return Lse{ef * kLn2High, fmaf(__log2f(f), kLn2, ef * kLn2Low)};
+}
+
+__device__ __forceinline__ Lse lse_of(float m, const Lse& ln_s) {
+    float err;
+    const float hi = add_with_error(m, ln_s.hi, err);
+    return Lse{hi, ln_s.lo + fmaf(-ref_error(m), kLn2, err)};
+}
+
+// z - lse, rounded once where it is finite; not above 0, by which the sum's own
+// rounding can pass it where one logit has all the weight.
+__device__ __forceinline__ float minus_lse(float z, const Lse& lse) {
+    float err;
+    const float d = add_with_error(z, -lse.hi, err);
+    const float lp = d + ((isfinite(d) ? err : 0.f) - lse.lo);
+    return lp > 0.f ? 0.f : lp;
 }
 
 // How a row of V logits is streamed: `head` elements up to the first 128-byte

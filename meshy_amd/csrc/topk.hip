@@ -235,7 +235,7 @@ __device__ __forceinline__ void forget(v4u (&v)[G]) {
 // ok set.
 template <int G, class OkF>
 __device__ __forceinline__ float maxima_and_sum(const v4u (&v)[G], float m, OkF ok, float (&cm)[G]) {
-    const float nm = -m * kLog2e;
+    const float nm = ref(m);
     float s0 = 0.f, s1 = 0.f;
 #pragma unroll
     for (int g = 0; g < G; ++g) {
@@ -296,12 +296,16 @@ __device__ __forceinline__ void set_floor(WaveBuf<CAP>& w, float lane_max, bool 
     }
 }
 
+// Of a tile, against a reference that stays: an element 14 above it has its
+// exponent rounded at the size of 20, 1e-6 of the sum.
+constexpr float kMaxSum = 0x1p20f;
+
 // One tile of G chunks per thread, those with ok set; the thread's first
 // starts at column col and the others NT chunks apart.  Its part of the
 // log-sum-exp, the row's floor if it is the first, and the chunks that reach
-// the threshold.  Past a lane's first tile the sum is taken against its
-// running max as it stands (rowstream.h, accumulate_at); where that overflows,
-// the max is raised first.
+// the threshold.  The sum is taken against the wave's maximum of the first tile
+// as it stands (rowstream.h, accumulate_at); where an element lies 14 above it,
+// the lane's reference is raised first.
 // Returns false, with no chunk appended, when the buffer has no room for them
 // all; collect() then takes the tile.
 template <int NT, int CAP, int G, class OkF>
@@ -310,13 +314,13 @@ __device__ __forceinline__ bool topk_tile(v4u (&v)[G], OkF ok, int32_t col, bool
     float t = 0.f;
     if (first) {
         const float tm = max_of(v, ok);
-        raise_max(m, s, t, tm);
+        raise_max(m, s, t, wave_max(tm));
         set_floor<NT>(w, tm, ok(0), k);
         forget(v);
     }
     float cm[G];
     float st = maxima_and_sum(v, m, ok, cm);
-    if (!(st <= 0x1p64f)) {
+    if (!(st <= kMaxSum)) {
         forget(v);
         raise_max(m, s, t, max_of(v, ok));
         forget(v);
@@ -350,7 +354,7 @@ __global__ __launch_bounds__(NT) void k_topk_vec(const uint16_t* __restrict__ lo
     __shared__ uint16_t s_key[kKeyRows][kWave];  // the waves' chunks, then the row's head and tail elements
     __shared__ uint64_t s_list[kMaxListed];
     __shared__ int s_listed;
-    __shared__ double s_lse;
+    __shared__ Lse s_lse;
     const int64_t r = blockIdx.x;
     const uint16_t* row = row_ptr(logits, r, T, stride_b, stride_t);
     const RowSpan sp = row_span(row, V);
@@ -467,10 +471,12 @@ __global__ __launch_bounds__(NT) void k_topk_vec(const uint16_t* __restrict__ lo
         // torch.logsumexp: NaN for a row holding NaN; otherwise +inf for a row
         // whose max is +inf (its candidates' log-probs are then NaN for the
         // +inf logit and -inf for finite ones), where s is NaN.
-        const double lse = __ballot(nan) ? __builtin_nan("") : m == __builtin_inff() ? __builtin_inf() : lse_of(m, s);
+        const Lse lse = __ballot(nan) ? Lse{__builtin_nanf(""), 0.f}
+                        : m == __builtin_inff() ? Lse{m, 0.f}
+                                                : lse_of(m, ln_of(s));
         if (tid == 0) {
             s_lse = lse;
-            if (lse_out) lse_out[r] = static_cast<float>(lse);
+            if (lse_out) lse_out[r] = lse.hi + lse.lo;
         }
     }
     __syncthreads();
@@ -518,7 +524,7 @@ __global__ __launch_bounds__(NT) void k_topk_vec(const uint16_t* __restrict__ lo
         __syncthreads();
     }
     const int listed = s_listed;
-    const double lse = s_lse;
+    const Lse lse = s_lse;
     for (int i = tid; i < listed; i += NT) {
         const uint64_t own = s_list[i];
         int rank = 0;
@@ -526,7 +532,7 @@ __global__ __launch_bounds__(NT) void k_topk_vec(const uint16_t* __restrict__ lo
         for (int j = 0; j < listed; ++j) rank += s_list[j] > own;
         if (rank < k) {
             ids[r * k + rank] = static_cast<int32_t>(~static_cast<uint32_t>(own));
-            lps[r * k + rank] = static_cast<float>(value_of(static_cast<uint32_t>(own >> 32)) - lse);
+            lps[r * k + rank] = minus_lse(value_of(static_cast<uint32_t>(own >> 32)), lse);
         }
     }
 }
