@@ -501,45 +501,69 @@ __global__ __launch_bounds__(kCountThreads) void k_gae_count(meshy_gae_args g, f
     if (cur >= 0 && cur <= g.n_docs && acc != 0.f) atomicAdd(cnt + cur, acc);
 }
 
-// Masked token count of document blockIdx.x over its offsets range: every
-// thread sums a fixed set of positions, then a fixed-order block sum; the
-// result does not depend on timing.  Bound by the longest documents, one
-// workgroup each: 16 positions per thread and step, in four 16-byte loads in
-// flight together (vec: the mask is 16-byte aligned), take 7.0 us for the 1024
-// documents of 6.35 M tokens, 11.9 with four 4-byte loads and 256 threads.
-constexpr int kDocCountThreads = 512;
-
-__global__ __launch_bounds__(kDocCountThreads) void k_gae_doc_count(const float* __restrict__ mask,
-                                                                    const int64_t* __restrict__ off, bool vec,
-                                                                    float* __restrict__ cnt) {
-    __shared__ float s_red[kDocCountThreads / kWave];
-    const int64_t d = blockIdx.x;
-    const int64_t lo = off[d];
-    const int64_t hi = off[d + 1];
-    const int tid = threadIdx.x;
-    // Groups of four positions [4 g0, 4 g1), and what lies before and after.
-    const int64_t g0 = vec ? (lo + 3) / 4 : hi;
-    const int64_t g1 = vec ? max(hi / 4, g0) : g0;
-    const int64_t head = vec ? min(4 * g0, hi) : hi;
+// The sum of the mask over [lo, hi), positions counted from the 16-byte boundary
+// at or before the mask (`base`), as NT threads share it: groups of four
+// positions with four 16-byte loads in flight per thread, and what lies before
+// and after the groups one by one.
+template <int NT>
+__device__ __forceinline__ float mask_sum(const float* __restrict__ base, int64_t lo, int64_t hi, int tid) {
+    const int64_t g0 = (lo + 3) / 4;
+    const int64_t g1 = max(hi / 4, g0);
+    const int64_t head = min(4 * g0, hi);
     float acc = 0.f;
     constexpr int kIn = 4;
-    for (int64_t g = g0 + tid; g < g1; g += kIn * kDocCountThreads) {
+    for (int64_t g = g0 + tid; g < g1; g += kIn * NT) {
         f32x4 m[kIn];
 #pragma unroll
-        for (int u = 0; u < kIn; ++u)
-            m[u] = *reinterpret_cast<const f32x4*>(mask + 4 * min(g + u * kDocCountThreads, g1 - 1));
+        for (int u = 0; u < kIn; ++u) m[u] = *reinterpret_cast<const f32x4*>(base + 4 * min(g + u * NT, g1 - 1));
 #pragma unroll
         for (int u = 0; u < kIn; ++u) {
             const float s = (m[u].x + m[u].y) + (m[u].z + m[u].w);
-            acc += g + u * kDocCountThreads < g1 ? s : 0.f;
+            acc += g + u * NT < g1 ? s : 0.f;
         }
     }
-    for (int64_t t = lo + tid; t < head; t += kDocCountThreads) acc += mask[t];
-    if (vec) {
-        for (int64_t t = max(4 * g1, head) + tid; t < hi; t += kDocCountThreads) acc += mask[t];
+    for (int64_t t = lo + tid; t < head; t += NT) acc += base[t];
+    for (int64_t t = max(4 * g1, head) + tid; t < hi; t += NT) acc += base[t];
+    return acc;
+}
+
+// Masked token counts over the documents' offset ranges: every thread sums a
+// fixed set of positions, then a fixed-order wave or block sum; the result does
+// not depend on timing.  With kDocs = 1 a workgroup takes a document: bound by
+// the longest, 7.0 us for the 1024 documents of 6.35 M tokens (11.9 with four
+// 4-byte loads and 256 threads).  Where that would be thousands of workgroups
+// for short documents (kManyDocs), one takes a document per wave, and then each
+// of them that is too long for a wave together: 65536 documents of 60 tokens, the
+// whole GAE call, 74 us against 141 with a workgroup each (82 of 256 threads).
+constexpr int kDocCountThreads = 512;
+constexpr int kManyDocs = 2048;
+constexpr int64_t kWaveDocTokens = 8192;
+
+template <int kDocs>
+__global__ __launch_bounds__(kDocCountThreads) void k_gae_doc_count(const float* __restrict__ base, int shift,
+                                                                    const int64_t* __restrict__ off, int64_t n_docs,
+                                                                    float* __restrict__ cnt) {
+    static_assert(kDocs == 1 || kDocs == kDocCountThreads / kWave, "a wave per document");
+    __shared__ float s_red[kDocCountThreads / kWave];
+    const int64_t d0 = static_cast<int64_t>(blockIdx.x) * kDocs;
+    if constexpr (kDocs > 1) {
+        const int64_t d = d0 + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+        if (d < n_docs) {
+            const int64_t lo = off[d], hi = off[d + 1];
+            if (hi - lo <= kWaveDocTokens) {
+                const int lane = threadIdx.x % kWave;
+                const float acc = wave_sum(mask_sum<kWave>(base, lo + shift, hi + shift, lane));
+                if (lane == 0) cnt[d] = acc;
+            }
+        }
     }
-    acc = block_sum<kDocCountThreads>(acc, s_red);
-    if (tid == 0) cnt[d] = acc;
+    for (int64_t d = d0; d < min(d0 + kDocs, n_docs); ++d) {
+        const int64_t lo = off[d], hi = off[d + 1];
+        if (kDocs > 1 && hi - lo <= kWaveDocTokens) continue;
+        const float acc = block_sum<kDocCountThreads>(
+            mask_sum<kDocCountThreads>(base, lo + shift, hi + shift, static_cast<int>(threadIdx.x)), s_red);
+        if (threadIdx.x == 0) cnt[d] = acc;
+    }
 }
 
 // The thread's maps (contiguous positions) folded right to left.
@@ -953,8 +977,14 @@ int gae_launch(const meshy_gae_args& g, hipStream_t stream) {
     // Document lengths only matter for lambda (advantages / lam_doc), not for returns.
     if (!g.lengths && (g.adv || g.lam_doc) && g.seg_offsets) {
         if (g.n_docs > 0) {
-            hipLaunchKernelGGL(k_gae_doc_count, dim3(static_cast<unsigned>(g.n_docs)), dim3(kDocCountThreads), 0,
-                               stream, g.mask, g.seg_offsets, reinterpret_cast<uintptr_t>(g.mask) % 16 == 0, ws.cnt);
+            const int shift = static_cast<int>(reinterpret_cast<uintptr_t>(g.mask) % 16 / sizeof(float));
+            auto count = [&](auto kernel, int docs) {
+                hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(ceil_div(g.n_docs, docs))),
+                                   dim3(kDocCountThreads), 0, stream, g.mask - shift, shift, g.seg_offsets, g.n_docs,
+                                   ws.cnt);
+            };
+            if (g.n_docs > kManyDocs) count(k_gae_doc_count<kDocCountThreads / kWave>, kDocCountThreads / kWave);
+            else count(k_gae_doc_count<1>, 1);
             if ((rc = check_launch("meshy_gae(count)"))) return rc;
         }
     } else if (!g.lengths && (g.adv || g.lam_doc)) {

@@ -1,9 +1,10 @@
 """The masked document lengths that GAE counts from segment offsets.
 
 The count reads groups of four positions with 16-byte loads, 8192 per step,
-and what lies before and after them one by one.  Documents start at every
-offset modulo 4 and have the lengths around those edges, empty ones among
-them; a mask that is not 16-byte aligned is read one by one.  Counts of 0/1
+and what lies before and after them one by one, wherever the mask starts.
+Documents start at every offset modulo 4 and have the lengths around those edges,
+empty ones among them; with more than 2048 documents a wave takes one, and those
+beyond 8192 tokens go to whole workgroups.  Counts of 0/1
 masks are exact (lambda equals the fp32 formula of the exact count); sums of
 fractional masks, up to 2^14 terms of at most 1 in fp32, lie within 2^-20
 relative of float64, and lambda within that of 1 / (alpha L).
@@ -44,3 +45,21 @@ def test_lambda_of_counted_lengths(dev, lead, offset, fractional):
         assert (err <= 2.0 ** -20 / counted.clamp(min=1) + 2.0 ** -23).all()
     else:
         assert torch.equal(lam.cpu(), _lambda(counted.float()))
+
+
+@pytest.mark.parametrize("n", [2048, 2049, 2055, 9001])
+@pytest.mark.parametrize("offset", [0, 1, 3])
+def test_lambda_of_many_documents(dev, n, offset):
+    from meshy_amd.gae import gae_and_returns
+
+    g = torch.Generator().manual_seed(n + offset)
+    lengths = torch.randint(0, 40, (n,), generator=g)
+    lengths[[0, 7, n // 2, n - 1]] = torch.tensor([8192, 8193, 40000, 16411])  # a wave's last, and workgroups'
+    total = int(lengths.sum())
+    doc = torch.repeat_interleave(torch.arange(n), lengths)
+    flat = (torch.rand(total + offset, generator=g) < 0.7).float()
+    mask = flat.to(dev)[offset:].view(1, total)
+    zeros = torch.zeros(1, total, device=dev)
+    _, _, lam = gae_and_returns(zeros, zeros, mask, doc.view(1, -1).to(dev), n)
+    counted = torch.zeros(n, dtype=torch.float64).index_add_(0, doc, flat[offset:].double())
+    assert torch.equal(lam.cpu(), _lambda(counted.float()))
