@@ -700,8 +700,9 @@ __global__ __launch_bounds__(NT) void k_lp_bwd_any(BwdArgs a) {
 }
 
 // 16-byte loads in flight per thread per tile, for the rows that fill several
-// tiles and for the others (their last tile is predicated and rounds up).
-constexpr int kFwdUnroll = 8, kFwdShortUnroll = 2;
+// tiles, for middle ones and for the others (the last tile is predicated and
+// rounds up).
+constexpr int kFwdUnroll = 8, kFwdMidUnroll = 3, kFwdShortUnroll = 2;
 constexpr int kBwdThreads = 256;
 constexpr int kBwdUnroll = 2;
 // Below this a wave of the flat pass holds several rows and waits for the
@@ -741,10 +742,12 @@ int check_common(const void* logits, int64_t rows, int64_t T, int64_t V, int64_t
 // undivided rows of 151936 logits, 256 threads 19.1.  From 2048 rows on, long
 // rows (3 full tiles and more) stream fastest with those too (16384 rows of
 // 151936: 703 us against 714 with 256 threads; 4096: 181 against 184 with 2
-// loads).  All others take the registers of 2 loads and 8 waves per SIMD, in
+// loads).  All others take the registers of 2 or 3 loads and 8 waves per SIMD, in
 // fewer threads where a short row would leave them idle, as long as the rows
 // still fill the CUs (128 threads: 16 workgroups per CU, 4096 in all):
-//   4096 rows of 65537 logits    512 x 2: 80 us   256 x 2: 82   256 x 8: 83
+//   4206 rows of 50257 logits    512 x 3: 67 us   512 x 2: 68   256 x 8: 67
+//   2048 rows of 50257           512 x 3: 33      512 x 2: 35   256 x 8: 35
+//   4096 rows of 65537           512 x 3: 80      512 x 2: 80   256 x 8: 83
 //   4096 rows of 32768           512 x 2: 42      256 x 2: 43   256 x 8: 43
 //   4096 rows of 16384           256 x 2: 23      512 x 2: 24   256 x 8: 25
 //   1024 rows of 24576           512 x 2: 9.9     256 x 2: 10.3 256 x 8: 11.2
@@ -760,7 +763,8 @@ struct FwdShape {
 FwdShape fwd_shape(int64_t n, int64_t V, int n_ids) {
     if (n <= 256 || (n >= 2048 && V >= 3 * 512 * kFwdUnroll * 8)) return {512, kFwdUnroll};
     if (V <= 1024 || (n_ids <= 128 && (V <= 4096 || (V <= 8192 && n >= 4096)))) return {128, kFwdShortUnroll};
-    return {V < 32768 && n > 1024 ? 256 : 512, kFwdShortUnroll};
+    const bool mid = V >= 3 * 512 * kFwdMidUnroll * 8 && V < 3 * 512 * kFwdUnroll * 8;
+    return {V < 32768 && n > 1024 ? 256 : 512, mid ? kFwdMidUnroll : kFwdShortUnroll};
 }
 
 // Workgroups per row.  One workgroup to a row is bound by its CU's exponentials
@@ -806,6 +810,7 @@ int launch_fwd(const uint16_t* logits, int64_t rows, int64_t T, int64_t V, int64
                            out, entropy, lse, Split{});
     };
     if (shape.unroll == kFwdUnroll) go(k_lpe_fwd_vec<512, kFwdUnroll, false>);
+    else if (shape.unroll == kFwdMidUnroll) go(k_lpe_fwd_vec<512, kFwdMidUnroll, false>);
     else if (shape.threads == 512) go(k_lpe_fwd_vec<512, kFwdShortUnroll, false>);
     else if (shape.threads == 256) go(k_lpe_fwd_vec<256, kFwdShortUnroll, false>);
     else go(k_lpe_fwd_vec<128, kFwdShortUnroll, false>);

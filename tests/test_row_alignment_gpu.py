@@ -63,7 +63,8 @@ def test_forward_on_both_sides_of_the_workgroup_size_rule(dev, T, V):
 # Both sides of the bounds on rows, logits and ids that choose a workgroup's
 # threads and loads for short and middle rows.
 @pytest.mark.parametrize("T,V,K", [(257, 1024, 256), (257, 1025, 128), (257, 1025, 129), (257, 4097, 256), (4095, 8192, 9),
-                                   (4096, 8192, 200), (4096, 8193, 9), (1024, 20001, 9), (1025, 20001, 9), (1025, 32767, 9), (1025, 32768, 9), (257, 131073, 200)])
+                                   (4096, 8192, 200), (4096, 8193, 9), (1024, 20001, 9), (1025, 20001, 9), (1025, 32767, 9), (1025, 32768, 9), (300, 36863, 9), (300, 36864, 9),
+                                   (300, 98303, 9), (257, 131073, 200)])
 def test_gather_on_both_sides_of_the_shape_rules(dev, T, V, K):
     from meshy_amd import logprob, topk
 
