@@ -114,6 +114,7 @@ class _Layout:
     def __init__(self) -> None:
         self.size = 0
         self.regions: dict[str, tuple[int, int, torch.dtype]] = {}
+        self.token_specs: tuple = ()  # of a pack's outputs: token_views' regions
 
     def add(self, name: str, n: int, dtype: torch.dtype) -> None:
         nbytes = n * (_ITEMSIZE.get(dtype) or dtype.itemsize)
@@ -656,6 +657,9 @@ def _out_layout(n_out: int, n_docs_total: int, n_micro: int, rollout_lp: bool, a
     if teacher_k:
         out_lay.add("teacher_ids", n_out * teacher_k, torch.int64)
         out_lay.add("teacher_lps", n_out * teacher_k, torch.float32)
+    regions = out_lay.regions
+    out_lay.token_specs = tuple((regions[name][0], _SCALAR_TYPE[regions[name][2]]) if name in regions else None
+                                for name in _PackViews._TOK)
     if len(_OUT_LAYOUTS) >= 4096:
         _OUT_LAYOUTS.clear()
     _OUT_LAYOUTS[key] = out_lay
@@ -848,11 +852,8 @@ class _PackViews:
 
     def _token_views(self) -> list:
         if self._tok is None:
-            regions = self.out_lay.regions
-            specs = tuple((regions[name][0], _SCALAR_TYPE[regions[name][2]]) if name in regions else None
-                          for name in self._TOK)
             rows, seq = (np.asarray(x, np.int64).tobytes() for x in (self._job.rows, self._job.seq))
-            self._tok = _lib.stage().token_views(self.obuf, specs, rows, seq, self.n_out)
+            self._tok = _lib.stage().token_views(self.obuf, self.out_lay.token_specs, rows, seq, self.n_out)
         return self._tok
 
     def tokens(self, mb: "PackedBatch", f: dict) -> None:
